@@ -171,7 +171,8 @@ __global__ void k_hs_derivatives(const float* __restrict__ frames,
 // tile plus an R-pixel halo of U, V, fx, fy, ft is loaded once; sub-iteration s updates the
 // cells within iters - s of the tile (their 3 x 3 neighbours were updated by sub-iteration
 // s - 1), so after `iters` sub-iterations the tile holds the exact iterate.  A neighbour outside
-// the image is the nearest edge cell (mode 'reflect' at distance 1).
+// the image is the nearest edge cell (mode 'reflect' at distance 1).  Used for float32 flows,
+// which round uAvg and every later operation to float32; float64 flows run on k_hs_strips.
 //
 //   uAvg = sum of the 8 neighbours x HSKERN (scipy's raster order, float64, rounded to T)
 //   der  = ((fx uAvg + fy vAvg) + ft) / den,   den = (float)((alpha^2 + fx^2) + fy^2)
@@ -273,6 +274,181 @@ __global__ __launch_bounds__(NT) void k_hs_iterate(
       Vout[g] = sV[c];
     }
   }
+}
+
+// Float64 iterations on register strips.  A wave owns S rows x 64 C columns of one frame pair
+// (each lane C neighbouring columns) and keeps U, V and the scaled derivatives
+//   (gx, gy, gt) = (fx, fy, ft) / sqrt(den)
+// in registers for `iters` iterations, so that
+//   U = uAvg - gx d,  V = vAvg - gy d,  d = (gx uAvg + gy vAvg) + gt
+// needs no division.  HSKERN separates: with p(x) = w2 c + w1 a, a = up + down and c the cell
+// itself, uAvg = w2 a(x) + p(x - 1) + p(x + 1), so one value per cell crosses to each side: by a
+// register move between a lane's own columns, by a DPP wave shift at the lane's edge.  Rows
+// cross between waves through LDS, two per wave and iteration (double buffered, one barrier).
+// NW waves stack to a band of NW S rows.  A band that does not hold the whole image keeps a halo
+// of `iters` rows (and columns) on each open side, whose cells go stale one per iteration.
+//
+// Bound: float64 issue (16 float64 instructions and 4 to 8 register moves per cell and iteration)
+// and, between launches, 44 B per pixel of U, V, fx, fy, ft.  Eight cells per lane at 10
+// registers each leave four waves per SIMD, which hide the barrier and the row exchange: 640
+// pairs of 128 x 128, 200 iterations take 3.78 ms (16 cells and two waves per SIMD: 3.96; the
+// LDS-tile form above, which reads 16 float64 neighbours per cell from LDS and divides: 11.6).
+// Two columns per lane halve the DPP moves (one column: 4.08 ms), one suits narrow images; three
+// (5 rows, 40-row bands) were slower at 128 columns (6.9 ms) and at 160 (9.2 against 8.7).
+constexpr int kHsWaves = 16;
+constexpr int hs_strip_rows(int cols) { return 8 / cols; }
+
+// nx x ny tiles of an image.  Along a side with several tiles, tile i loads from cell i ow on; it
+// writes from halo cells further on (the first tile from the image's edge) up to the next tile's
+// first written cell (the last tile up to the image's edge).  With one tile ow is unused.  halo: iterations per launch (0: one tile holds the image).
+struct HsTiling {
+  int nx, ny;
+  int ow, oh;
+  int halo;
+};
+
+template <int C, int S>
+__global__ __launch_bounds__(kHsWaves * 64) void k_hs_strips(
+    const float* __restrict__ gfx, const float* __restrict__ gfy, const float* __restrict__ gft,
+    int H, int W, HsTiling t, float alpha2, int iters, const double* Uin, const double* Vin,
+    double* Uout, double* Vout) {
+#pragma clang fp contract(off)
+  constexpr int NW = kHsWaves, LW = 64 * C;
+  __shared__ double rows[2][NW][2][2][LW];   // parity, wave, top / bottom row, U / V, column
+  const int tile = (int)(blockIdx.x % (unsigned)(t.nx * t.ny));
+  const int64_t base = (int64_t)(blockIdx.x / (unsigned)(t.nx * t.ny)) * H * W;
+  const int tx = tile % t.nx, ty = tile / t.nx;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int x0 = tx * t.ow + lane * C, yw = ty * t.oh + w * S;
+  double U[S][C], V[S][C], gx[S][C], gy[S][C], gt[S][C];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      // cells outside the image are loaded as its edge cells; they reach no cell inside
+      const int64_t g = base + (int64_t)min(yw + s, H - 1) * W + min(x0 + j, W - 1);
+      U[s][j] = Uin[g];
+      V[s][j] = Vin[g];
+      const float fx = gfx[g], fy = gfy[g], ft = gft[g];
+      const float den = (alpha2 + fx * fx) + fy * fy;
+      const double r = rsqrt((double)den);
+      gx[s][j] = fx * r;
+      gy[s][j] = fy * r;
+      gt[s][j] = ft * r;
+    }
+  }
+  // Columns beyond the image pass zero to their neighbours (their weights are zero), the wave's
+  // outer lanes read zero past its ends, and a column at the image's edge adds its own p (edge)
+  // for the neighbour it lacks.
+  double w1[C], w2[C], edge[C];
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    w1[j] = x0 + j < W ? 1.0 / 12 : 0.0;
+    w2[j] = x0 + j < W ? 1.0 / 6 : 0.0;
+    edge[j] = (x0 + j == 0 ? 1.0 : 0.0) + (x0 + j == W - 1 ? 1.0 : 0.0);
+  }
+  const int s_last = H - 1 - yw;             // the image's last row within the strip
+  // row s from the rows above and below it
+  auto update = [&](int s, const double* up_u, const double* up_v, const double* dn_u,
+                    const double* dn_v) {
+    double au[C], av[C], qu[C], qv[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      au[j] = up_u[j] + dn_u[j];
+      av[j] = up_v[j] + dn_v[j];
+      qu[j] = fma(w1[j], au[j], w2[j] * U[s][j]);
+      qv[j] = fma(w1[j], av[j], w2[j] * V[s][j]);
+    }
+    const double lu = dpp_move<0x138, 0xf>(qu[C - 1]);             // wave_shr:1
+    const double lv = dpp_move<0x138, 0xf>(qv[C - 1]);
+    const double ru = dpp_move<0x130, 0xf>(qu[0]);                 // wave_shl:1
+    const double rv = dpp_move<0x130, 0xf>(qv[0]);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const double l_u = j == 0 ? lu : qu[j > 0 ? j - 1 : 0];
+      const double l_v = j == 0 ? lv : qv[j > 0 ? j - 1 : 0];
+      const double r_u = j == C - 1 ? ru : qu[j < C - 1 ? j + 1 : j];
+      const double r_v = j == C - 1 ? rv : qv[j < C - 1 ? j + 1 : j];
+      const double ua = fma(edge[j], qu[j], fma(1.0 / 6, au[j], l_u) + r_u);
+      const double va = fma(edge[j], qv[j], fma(1.0 / 6, av[j], l_v) + r_v);
+      const double d = fma(gx[s][j], ua, fma(gy[s][j], va, gt[s][j]));
+      U[s][j] = fma(-gx[s][j], d, ua);
+      V[s][j] = fma(-gy[s][j], d, va);
+    }
+    __builtin_amdgcn_sched_barrier(0);       // row by row: interleaved rows overflow the registers
+  };
+  for (int it = 0; it < iters; ++it) {
+    double(*rb)[2][2][LW] = rows[it & 1];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      rb[w][0][0][j * 64 + lane] = U[0][j];
+      rb[w][0][1][j * 64 + lane] = V[0][j];
+      rb[w][1][0][j * 64 + lane] = U[S - 1][j];
+      rb[w][1][1][j * 64 + lane] = V[S - 1][j];
+    }
+    // the row below the image's last one repeats it
+#pragma unroll
+    for (int s = 0; s + 1 < S; ++s)
+      if (s == s_last) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+          U[s + 1][j] = U[s][j];
+          V[s + 1][j] = V[s][j];
+        }
+      }
+    __syncthreads();
+    double pu[C], pv[C], nu[C], nv[C];       // the row above; the row below the strip
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      // the first wave's strip starts at the image's top or in the halo, the last one's ends at
+      // its bottom or in the halo
+      const bool top = w == 0, bottom = w == NW - 1 || s_last == S - 1;
+      pu[j] = top ? U[0][j] : rb[top ? w : w - 1][1][0][j * 64 + lane];
+      pv[j] = top ? V[0][j] : rb[top ? w : w - 1][1][1][j * 64 + lane];
+      nu[j] = bottom ? U[S - 1][j] : rb[w + 1 < NW ? w + 1 : w][0][0][j * 64 + lane];
+      nv[j] = bottom ? V[S - 1][j] : rb[w + 1 < NW ? w + 1 : w][0][1][j * 64 + lane];
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      double cu[C], cv[C];
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        cu[j] = U[s][j];
+        cv[j] = V[s][j];
+      }
+      if (s + 1 < S) update(s, pu, pv, U[s + 1 < S ? s + 1 : s], V[s + 1 < S ? s + 1 : s]);
+      else update(s, pu, pv, nu, nv);
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        pu[j] = cu[j];
+        pv[j] = cv[j];
+      }
+    }
+  }
+  const int ox = tx ? tx * t.ow + t.halo : 0, oy = ty ? ty * t.oh + t.halo : 0;
+  const int ex = tx == t.nx - 1 ? W : (tx + 1) * t.ow + t.halo;
+  const int ey = ty == t.ny - 1 ? H : (ty + 1) * t.oh + t.halo;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int x = x0 + j, y = yw + s;
+      if (x >= ox && x < ex && y >= oy && y < ey) {
+        const int64_t g = base + (int64_t)y * W + x;
+        Uout[g] = U[s][j];
+        Vout[g] = V[s][j];
+      }
+    }
+}
+
+// Tiles of one side: n tiles of `cap` cells with a halo of R on each open side cover L cells when
+// L <= n cap - 2 (n - 1) R (the two end tiles have one open side each).  The largest such R for
+// n tiles, at most `niter`.
+inline int hs_halo(int L, int cap, int n, int niter) {
+  if (n == 1) return L <= cap ? niter : 0;
+  const int64_t r = ((int64_t)n * cap - L) / (2 * (n - 1));
+  return (int)std::max<int64_t>(0, std::min<int64_t>({r, (cap - 1) / 2, niter}));
 }
 
 // --- flow sum, orientation, magnitude (OpticalFlowMovie.py:21-24, 519-555) ----------------------
@@ -462,20 +638,57 @@ int memi_hs_iterate(const float* fx, const float* fy, const float* ft, int64_t n
   MEMI_CHECK_ARG(nP >= 0 && H >= 1 && W >= 1 && niter >= 0, "memi_hs_iterate: bad sizes");
   MEMI_CHECK_ARG(tmpU != U && tmpV != V && tmpU != tmpV && U != V,
                  "memi_hs_iterate: U, V, tmpU, tmpV must be distinct");
-  const int tiles_x = (W + kHsTile - 1) / kHsTile;
-  const int tiles_y = (H + kHsTile - 1) / kHsTile;
-  const int ntiles = tiles_x * tiles_y;
-  MEMI_CHECK_ARG(nP * ntiles < 0x7fffffffLL, "memi_hs_iterate: too many tiles");
   if (nP == 0 || niter == 0) return MEMI_OK;
-  const int launches = (niter + kHsHalo - 1) / kHsHalo;
-  const size_t bytes = (size_t)nP * H * W * (is_f64 ? 8 : 4);
   hipStream_t s = (hipStream_t)stream;
-  // ping-pong so that the last launch writes U, V
+  // numpy adds the Python float alpha**2 to a float32 array as float32
+  const float alpha2 = (float)(alpha * alpha);
+  int launches, step;
+  HsTiling t{};
+  int cols = 0;                      // columns per lane of the strip kernel (float64)
+  if (is_f64) {
+    // the shape and tile counts of least cost: cells computed per iteration, halos included
+    // (one column per lane: a tenth more per cell), plus, per launch, the pixels' traffic (44 B
+    // at ~8 B per CU cycle, about 18 cells' worth of issue)
+    double best = 0.0;
+    for (int c = 1; c <= 2; ++c) {
+      const int cap_x = 64 * c, cap_y = kHsWaves * hs_strip_rows(c);
+      const int nx0 = (W + cap_x - 1) / cap_x, ny0 = (H + cap_y - 1) / cap_y;
+      for (int nx = nx0; nx <= nx0 + 2 + nx0 / 4; ++nx)
+        for (int ny = ny0; ny <= ny0 + 3 + ny0 / 4; ++ny) {
+          const int R = std::min(hs_halo(W, cap_x, nx, niter), hs_halo(H, cap_y, ny, niter));
+          if (R < 1) continue;
+          const int l = (niter + R - 1) / R;
+          const double cost = (c == 1 ? 1.1 : 1.0) * nx * ny * cap_x * cap_y * niter +
+                              18.0 * l * H * W;
+          if (cols == 0 || cost < best) {
+            best = cost;
+            cols = c;
+            const int h = (niter + l - 1) / l;           // the iterations spread evenly
+            t.nx = nx;
+            t.ny = ny;
+            t.halo = nx * ny == 1 ? 0 : h;
+            t.ow = cap_x - 2 * h;
+            t.oh = cap_y - 2 * h;
+          }
+        }
+    }
+    step = t.halo ? t.halo : niter;
+  } else {
+    t.nx = (W + kHsTile - 1) / kHsTile;
+    t.ny = (H + kHsTile - 1) / kHsTile;
+    step = kHsHalo;
+  }
+  launches = (niter + step - 1) / step;
+  const int64_t ntiles = (int64_t)t.nx * t.ny;
+  MEMI_CHECK_ARG(nP * ntiles < 0x7fffffffLL, "memi_hs_iterate: too many tiles");
+  const size_t bytes = (size_t)nP * H * W * (is_f64 ? 8 : 4);
+  // ping-pong so that the last launch writes U, V (one launch of whole images works in place)
+  const bool in_place = is_f64 && ntiles == 1;
   void* cur_u = U;
   void* cur_v = V;
-  void* nxt_u = tmpU;
-  void* nxt_v = tmpV;
-  if (launches % 2) {
+  void* nxt_u = in_place ? U : tmpU;
+  void* nxt_v = in_place ? V : tmpV;
+  if (!in_place && launches % 2) {
     if (hipMemcpyAsync(tmpU, U, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess ||
         hipMemcpyAsync(tmpV, V, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess) {
       set_error("memi_hs_iterate: copy failed");
@@ -484,22 +697,27 @@ int memi_hs_iterate(const float* fx, const float* fy, const float* ft, int64_t n
     std::swap(cur_u, nxt_u);
     std::swap(cur_v, nxt_v);
   }
-  // numpy adds the Python float alpha**2 to a float32 array as float32
-  const float alpha2 = (float)(alpha * alpha);
   const dim3 grid((unsigned)(nP * ntiles));
   for (int l = 0, done = 0; l < launches; ++l) {
-    const int it = std::min(kHsHalo, niter - done);
-    if (is_f64)
-      hipLaunchKernelGGL((k_hs_iterate<double, kHsTile, kHsHalo, kHsThreads>), grid,
-                         dim3(kHsThreads), 0, s, fx, fy, ft, H, W, tiles_x, ntiles, alpha2, it,
-                         (const double*)cur_u, (const double*)cur_v, (double*)nxt_u,
-                         (double*)nxt_v);
-    else
+    const int it = std::min(step, niter - done);
+    if (is_f64) {
+      const dim3 block(kHsWaves * 64);
+      const double *ui = (const double*)cur_u, *vi = (const double*)cur_v;
+      double *uo = (double*)nxt_u, *vo = (double*)nxt_v;
+      if (cols == 1)
+        hipLaunchKernelGGL((k_hs_strips<1, hs_strip_rows(1)>), grid, block, 0, s, fx, fy, ft, H,
+                           W, t, alpha2, it, ui, vi, uo, vo);
+      else
+        hipLaunchKernelGGL((k_hs_strips<2, hs_strip_rows(2)>), grid, block, 0, s, fx, fy, ft, H,
+                           W, t, alpha2, it, ui, vi, uo, vo);
+      MEMI_CHECK_LAUNCH("k_hs_strips");
+    } else {
       hipLaunchKernelGGL((k_hs_iterate<float, kHsTile, kHsHalo, kHsThreads>), grid,
-                         dim3(kHsThreads), 0, s, fx, fy, ft, H, W, tiles_x, ntiles, alpha2, it,
+                         dim3(kHsThreads), 0, s, fx, fy, ft, H, W, t.nx, (int)ntiles, alpha2, it,
                          (const float*)cur_u, (const float*)cur_v, (float*)nxt_u,
                          (float*)nxt_v);
-    MEMI_CHECK_LAUNCH("k_hs_iterate");
+      MEMI_CHECK_LAUNCH("k_hs_iterate");
+    }
     std::swap(cur_u, nxt_u);
     std::swap(cur_v, nxt_v);
     done += it;

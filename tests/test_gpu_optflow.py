@@ -101,6 +101,34 @@ def test_hs_op_matches_oracle(cuda, H, W, niter):
     np.testing.assert_allclose(V, Vr, rtol=0, atol=1e-9 * scale)
 
 
+@pytest.mark.parametrize("H,W", [(1, 1), (2, 63), (65, 64), (63, 65), (64, 128), (129, 127),
+                                 (40, 129), (41, 192), (70, 193), (130, 130), (200, 260)])
+def test_hs_strips_match_direct_iteration(cuda, H, W):
+    """The float64 iterations on register strips at the edges of their tiles (sides below, at and
+    above 64, 128 and 192 columns, 40, 64 and 128 rows, several tiles each way), with large
+    gradients, against the plain iteration.  uAvg is a weighted mean and the update contracts, so
+    rounding (about 20 operations a step) adds up at most linearly: 37 x 20 x 1.1e-16 < 1e-13 of
+    the flow's scale."""
+    from scipy.ndimage import convolve
+    from manifoldem_python_amd import optflow
+    rng = np.random.default_rng(H * 1000 + W)
+    nP, niter = 3, 37
+    fx, fy, ft = (rng.normal(size=(3, nP, H, W)) * 3).astype(np.float32)
+    U0, V0 = rng.normal(size=(2, nP, H, W))
+    U, V = optflow.hs_iterate(_dev(fx), _dev(fy), _dev(ft), 2.0, niter, _dev(U0), _dev(V0))
+    for p in range(nP):
+        u, v = U0[p], V0[p]
+        den = (np.float32(4.0) + fx[p] ** 2) + fy[p] ** 2
+        top = max(np.abs(u).max(), np.abs(v).max())
+        for _ in range(niter):
+            ua, va = convolve(u, of.HSKERN), convolve(v, of.HSKERN)
+            d = (fx[p] * ua + fy[p] * va + ft[p]) / den
+            u, v = ua - fx[p] * d, va - fy[p] * d
+            top = max(top, np.abs(u).max(), np.abs(v).max())
+        np.testing.assert_allclose(U[p].cpu().numpy(), u, rtol=0, atol=1e-13 * top)
+        np.testing.assert_allclose(V[p].cpu().numpy(), v, rtol=0, atol=1e-13 * top)
+
+
 def test_hs_float32_start(cuda):
     """A float32 initial flow keeps the iteration in float32, as numpy does."""
     from manifoldem_python_amd import hornschunck_simple as hs
