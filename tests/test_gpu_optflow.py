@@ -47,6 +47,41 @@ def test_anisodiff_matches_oracle(cuda, option):
     np.testing.assert_array_equal(one, mov)
 
 
+@pytest.mark.parametrize("shape", [(2, 7, 33, 31), (1, 1, 5, 4), (1, 3, 2, 1100), (3, 2, 40, 1),
+                                   (1, 40, 32, 32), (40, 3, 64, 33)])
+@pytest.mark.parametrize("option", [1, 2])
+def test_anisodiff_blocks_and_frame_pieces(cuda, shape, option):
+    """Pixels across the diffusion's blocks (rows that end inside one, a row longer than one) and
+    frames in one or several pieces, against the float32 update with the float64 exp rounded.
+    Every operation but the exp is the same float32 operation; an exp off by one float32 ulp
+    moves a voxel by at most gamma 2^-24 |flux| per face and step, 6 faces and 4 steps: below
+    2e-7 of the movie's scale."""
+    from manifoldem_python_amd import optflow
+    rng = np.random.default_rng(sum(shape))
+    mov = (60 * rng.normal(size=shape)).astype(np.float32)
+    got = optflow.anisodiff3(_dev(mov), 5, 50, 0.1, (5., 3., 3.), option).cpu().numpy()
+    f32 = np.float32
+    for m in range(shape[0]):
+        out = mov[m].copy()
+        for _ in range(4):
+            div = []
+            for ax, h in ((0, 5.0), (1, 3.0), (2, 3.0)):
+                d = np.zeros_like(out)
+                lo = [slice(None)] * 3
+                hi = [slice(None)] * 3
+                lo[ax], hi[ax] = slice(None, -1), slice(1, None)
+                d[tuple(lo)] = np.diff(out, axis=ax)
+                q = d / f32(50)
+                g = (np.exp(-(q * q).astype(np.float64)).astype(f32) if option == 1 else
+                     f32(1) / (f32(1) + q * q)) / f32(h)
+                fl = g * d
+                v = fl.copy()
+                v[tuple(hi)] -= fl[tuple(lo)]
+                div.append(v)
+            out = out + f32(0.1) * ((div[0] + div[1]) + div[2])
+        np.testing.assert_allclose(got[m], out, rtol=0, atol=2e-7 * np.abs(mov).max())
+
+
 def test_block_average_exact(cuda):
     from manifoldem_python_amd import _native as nat
     mov = _smooth_movie(2, 12, 9, 1).reshape(2, 12, 9, 9)
