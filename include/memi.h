@@ -73,7 +73,7 @@ typedef struct memi_plan_info {
   int32_t chunks;      /* K chunks per half (P or R: two operand segments)               */
   int32_t max_n;
   int32_t gram_tile;   /* side of the Gram's output tiles (128 or 256)                  */
-  int32_t reserved;
+  int32_t auto_split;  /* chunks chosen by memi_plan: an upper bound for short operands */
 } memi_plan_info;
 
 typedef struct memi_ctf_params {
@@ -216,9 +216,12 @@ int memi_image_moments(const float* img, int64_t n, int64_t npix, double* sum, d
  * plan_host is non-NULL (capacity plan_cap bytes >= info->plan_bytes) also write the tables:
  * PD descriptors with their offsets filled in, Gram work items over the gram_tile x gram_tile
  * upper-triangle tiles of every PD x 2 halves (P, R) x `chunks`, those upper tiles, the
- * 128 x 128 full tiles of the Stage-2 kernels and the row list.  gram_tile: 128 or 256.  The
+ * 128 x 128 full tiles of the Stage-2 kernels and the row list.  gram_tile: 128 or 256.
+ * chunks: 1..64, or MEMI_CHUNKS_AUTO (0) for a split of 2 or more chosen from the number of
+ * tiles (-c, c <= 64: of c or more, which bounds the length of a float32 sum).  The
  * caller copies the plan to device memory once and passes it to every batched entry point
  * below (plan_dev). */
+#define MEMI_CHUNKS_AUTO 0
 int memi_plan(const memi_pd_desc* pds_in_host, int npd, int chunks, int gram_tile,
               void* plan_host, int64_t plan_cap, memi_plan_info* info);
 
@@ -233,11 +236,12 @@ int memi_plan(const memi_pd_desc* pds_in_host, int npd, int chunks, int gram_til
  * like the operand).
  * Each half's K range (two segments of Khp elements, 64-byte steps) is split into
  * info->chunks chunks of ceil(2 steps / chunks) steps, the last one shorter; a chunk count
- * that leaves an empty chunk is rejected.
+ * that leaves an empty chunk is rejected.  A plan with an automatic split uses as many of its
+ * chunks as the K range fills.
  * variant: Gram kernel schedule, 0 = default; for 128-wide tiles (two workgroups per CU)
- * 1 = prefetch one K step through registers, 2 = prefetch two (the default), 3 = load each K
- * step straight into LDS (global_load_lds) during the previous step's MFMAs; 256-wide tiles
- * (one workgroup per CU, 128 x 64 per wave) take 1 (the default) or 3.  Every schedule gives
+ * 1 = prefetch one K step through registers, 2 = prefetch two, 3 = load each K step straight
+ * into LDS (global_load_lds) during the previous step's MFMAs (the default); 256-wide tiles
+ * (one workgroup per CU, 128 x 64 per wave) take 1 or 3 (the default).  Every schedule gives
  * the same D bit for bit.
  * ev_start / ev_stop: optional hipEvent_t recorded on `stream` right before and after the
  * MFMA Gram kernel (NULL: not recorded), for timing that kernel alone. */

@@ -17,6 +17,7 @@ LIB_PATH = os.path.join(_HERE, "lib", "libmemi.so")
 
 PREC_FP32 = 0
 PREC_SPLIT_BF16 = 1
+CHUNKS_AUTO = 0          # memi_plan picks the K split from the number of tiles (-c: at least c)
 FILTER_BUTTER = 1
 FILTER_GAUSS = 2
 FILTER_BSPLINE = 4
@@ -40,7 +41,7 @@ class PlanInfo(ctypes.Structure):
                 ("plan_bytes", c_i64), ("d_elems", c_i64), ("mask_words", c_i64),
                 ("list_elems", c_i64), ("ws_floats", c_i64), ("flag_cap", c_i64),
                 ("chunks", c_i32), ("max_n", c_i32), ("gram_tile", c_i32),
-                ("reserved", c_i32)]
+                ("auto_split", c_i32)]
 
 
 class CtfParams(ctypes.Structure):

@@ -30,7 +30,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));   // 16 staged bytes
 
-constexpr int TB_FIN = 2048;           // tile entries per finalize workgroup
+constexpr int FB = 32;                 // side of a finalize workgroup's block of tile entries
 constexpr int ROW_STEP = 64;           // bytes of one operand row per K step
 constexpr int LDS_ROW = 64;            // LDS row stride (bytes); 16-byte chunks swizzled
 
@@ -322,7 +322,8 @@ template <int PREC, class S, int DEPTH>
 __global__ __launch_bounds__(S::NT, S::OCC) void k_gram_tiles(
     const char* __restrict__ op_hi, const char* __restrict__ op_lo, int64_t Khp, int spc,
     int steps, const int32_t* __restrict__ items, int64_t n_items,
-    const memi_pd_desc* __restrict__ pds, float* __restrict__ ws) {
+    const memi_pd_desc* __restrict__ pds, float* __restrict__ ws,
+    int32_t* __restrict__ flag_count) {
   using Cfg = GramCfg<PREC>;
   constexpr int ES = Cfg::ESIZE;
   constexpr int NA = Cfg::NARR;
@@ -340,6 +341,7 @@ __global__ __launch_bounds__(S::NT, S::OCC) void k_gram_tiles(
   // items (consecutive items share operand panels and K ranges).  gridDim.x % 8 == 0.
   const int64_t q8 = gridDim.x / 8;
   const int64_t it = (int64_t)(blockIdx.x % 8) * q8 + blockIdx.x / 8;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flag_count = 0;   // for the finalize
   if (it >= n_items) return;
   const int32_t* itm = items + it * 6;
   const int pd = itm[0], ti = itm[1], tj = itm[2], half = itm[3], chunk = itm[4];
@@ -348,10 +350,11 @@ __global__ __launch_bounds__(S::NT, S::OCC) void k_gram_tiles(
   const int mi = min(BT, P.n - ti * BT);
   const int mj = min(BT, P.n - tj * BT);
   const int64_t row_bytes = 4 * Khp * ES;
-  // chunk c covers steps [c*spc, min((c+1)*spc, 2*steps)) of the half's two segments; the
-  // host guarantees none is empty
+  // chunk c covers steps [c*spc, min((c+1)*spc, 2*steps)) of the half's two segments; an
+  // automatic split may leave the last chunks empty (the finalize does not read those)
   const int s0 = chunk * spc;
   const int nks = min(spc, 2 * steps - s0);
+  if (nks <= 0) return;
 
   const int t = threadIdx.x;
   const int lane = t & 63, wv = t >> 6;
@@ -425,38 +428,72 @@ __global__ __launch_bounds__(S::NT, S::OCC) void k_gram_tiles(
     }
 }
 
-// Reduce the P and R partials of one upper tile in float64, write D and its mirror, and queue
-// entries with a large cancellation ratio for direct recomputation.  blockIdx.y: which
-// TB_FIN-entry part of the BT x BT tile this block reduces.
+// Reduce the P and R partials of one upper tile in float64 (in chunk order), write D and its
+// mirror, and queue entries with a large cancellation ratio for direct recomputation.
+// blockIdx.y: which FB x FB block of the BT x BT tile this workgroup reduces.  live: chunks that
+// hold steps, of the plan's `chunks`.
+//
+// Bound: the partials (2 live x 64 KB per 128-wide tile) and D.  Each thread sums four
+// neighbouring entries with the chunks' loads four at a time in flight (one entry per thread and
+// one chunk at a time cost ~4 us per chunk of memory latency at 10 tiles), and the mirror goes
+// through LDS so that both copies of D are written in whole lines.
 __global__ __launch_bounds__(256) void k_gram_finalize(const int32_t* __restrict__ utiles,
                                                        const memi_pd_desc* __restrict__ pds,
                                                        const float* __restrict__ ws, int chunks,
-                                                       int BT, double kappa,
+                                                       int live, int BT, double kappa,
                                                        float* __restrict__ D,
                                                        int32_t* __restrict__ flags,
                                                        int64_t flag_cap,
                                                        int32_t* __restrict__ flag_count) {
+  __shared__ float tr[FB][FB + 1];
   const int32_t* u = utiles + (int64_t)blockIdx.x * 4;
   const int pd = u[0], ti = u[1], tj = u[2];
   const int64_t slot0 = u[3];
   const memi_pd_desc P = pds[pd];
   const int n = P.n;
   const int64_t tile = (int64_t)BT * BT;
-  const int e0 = blockIdx.y * TB_FIN, e1 = e0 + TB_FIN;
-  for (int e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-    const int r = e / BT, c = e % BT;
-    const int i = ti * BT + r, j = tj * BT + c;
-    if (i >= n || j >= n) continue;
-    if (ti == tj && c < r) continue;
-    double d = 0.0;
-    if (i != j) {
-      double Pp = 0.0, R = 0.0;
-      for (int ch = 0; ch < chunks; ++ch) {
-        Pp += (double)ws[(slot0 + ch) * tile + e];
-        R += (double)ws[(slot0 + chunks + ch) * tile + e];
+  const int nb = BT / FB;
+  const int br = (int)blockIdx.y / nb, bc = (int)blockIdx.y % nb;
+  const int i0 = ti * BT + br * FB, j0 = tj * BT + bc * FB;
+  if (i0 >= n || j0 >= n || j0 + FB <= i0) return;      // no entry on or above the diagonal
+  const int r = threadIdx.x / (FB / 4), c4 = (threadIdx.x % (FB / 4)) * 4;
+  const int i = i0 + r;
+  const float* pp = ws + slot0 * tile + (br * FB + r) * BT + bc * FB + c4;
+  const float* pr = pp + chunks * tile;
+  double Pp[4] = {}, R[4] = {};
+  int ch = 0;
+  for (; ch + 4 <= live; ch += 4) {
+    floatx4_t a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      a[q] = *(const floatx4_t*)(pp + (ch + q) * tile);
+      b[q] = *(const floatx4_t*)(pr + (ch + q) * tile);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        Pp[e] += (double)a[q][e];
+        R[e] += (double)b[q][e];
       }
-      d = Pp - 2.0 * R;
-      if (Pp + 2.0 * fabs(R) > kappa * d) {
+  }
+  for (; ch < live; ++ch) {
+    const floatx4_t a = *(const floatx4_t*)(pp + ch * tile);
+    const floatx4_t b = *(const floatx4_t*)(pr + ch * tile);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      Pp[e] += (double)a[e];
+      R[e] += (double)b[e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int j = j0 + c4 + e;
+    const bool in = i < n && j < n && j >= i;
+    double d = 0.0;
+    if (in && i != j) {
+      d = Pp[e] - 2.0 * R[e];
+      if (Pp[e] + 2.0 * fabs(R[e]) > kappa * d) {
         const int32_t slot = atomicAdd(flag_count, 1);
         if (slot < flag_cap) {
           flags[3 * (int64_t)slot + 0] = pd;
@@ -465,8 +502,15 @@ __global__ __launch_bounds__(256) void k_gram_finalize(const int32_t* __restrict
         }
       }
     }
-    D[P.d_off + (int64_t)i * n + j] = (float)d;
-    if (i != j) D[P.d_off + (int64_t)j * n + i] = (float)d;
+    tr[r][c4 + e] = (float)d;
+    if (in) D[P.d_off + (int64_t)i * n + j] = (float)d;
+  }
+  __syncthreads();
+  const int jm = j0 + r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int im = i0 + c4 + e;
+    if (jm < n && im < n && jm > im) D[P.d_off + (int64_t)jm * n + im] = tr[c4 + e][r];
   }
 }
 
@@ -504,11 +548,29 @@ __global__ __launch_bounds__(256) void k_gram_recompute(const int32_t* __restric
   }
 }
 
-__global__ void k_zero_i32(int32_t* p, int64_t n) {
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * blockDim.x)
-    p[e] = 0;
+// K chunks per half (at least `least`) for `ut` upper tiles when the caller leaves the split open.
+// A launch runs ceil(2 ut c / slots) rounds of resident workgroups (two 128-wide ones per CU),
+// each 1 / c of a half long; every round adds its start and stores, every chunk partial tiles to
+// write and read.  The weights are the best of a grid over measured launches (Gram + finalize;
+// 1 to 738 tiles, 132 to 1040 K steps per half, c = 2 to 64): within 2 % of the best c on
+// average, 15 % at worst.  Times at c = 2 and at the rule's c: 1 tile, N = 64: 61, 20 us; 10 tiles,
+// N = 180: 440, 93; 36 tiles, N = 128: 231, 120; 136 tiles, N = 128: 566, 448.
+inline int auto_chunks(int64_t ut, int BT, int least) {
+  const double slots = BT == 256 ? 256.0 : 512.0;
+  const double area = BT == 256 ? 4.0 : 1.0;
+  int best = 0;
+  double cost = 0.0;
+  for (int c = least; c <= 64; ++c) {
+    const double rounds = std::ceil(2.0 * ut * c / slots);
+    const double f = rounds / c + 0.01 * rounds + c * (1e-4 * area * ut + 2e-4);
+    if (best == 0 || f < cost) {
+      cost = f;
+      best = c;
+    }
+  }
+  return best;
 }
+constexpr int kAutoMinSteps = 6;     // least K steps of a chunk of an automatic split
 
 }  // namespace memi
 
@@ -519,14 +581,14 @@ extern "C" {
 int memi_plan(const memi_pd_desc* pds_in, int npd, int chunks, int gram_tile,
               void* plan_host, int64_t plan_cap, memi_plan_info* info) {
   MEMI_CHECK_ARG(info != nullptr && (npd == 0 || pds_in != nullptr), "memi_plan: null pointer");
-  MEMI_CHECK_ARG(npd >= 0 && chunks >= 1 && chunks <= 64, "memi_plan: bad npd/chunks");
+  MEMI_CHECK_ARG(npd >= 0 && chunks >= -64 && chunks <= 64, "memi_plan: bad npd/chunks");
   MEMI_CHECK_ARG(gram_tile == 128 || gram_tile == 256,
                  "memi_plan: gram_tile must be 128 or 256 (got %d)", gram_tile);
   constexpr int FT = 128;             // side of the full-matrix tiles of the Stage-2 kernels
   const int BT = gram_tile;
   memi_plan_info I{};
   I.n_pd = npd;
-  I.chunks = chunks;
+  I.auto_split = chunks <= MEMI_CHUNKS_AUTO;
   I.gram_tile = BT;
   int64_t d = 0, mw = 0, le = 0, rows = 0, items = 0, ut = 0, ft = 0, fc = 0;
   int max_n = 0;
@@ -548,6 +610,8 @@ int memi_plan(const memi_pd_desc* pds_in, int npd, int chunks, int gram_tile,
     fc += n * (n - 1) / 2;
     if (n > max_n) max_n = (int)n;
   }
+  if (I.auto_split) chunks = auto_chunks(ut, BT, std::max(2, -chunks));
+  I.chunks = chunks;
   items = ut * 2 * chunks;
   MEMI_CHECK_ARG(items < (1LL << 31), "memi_plan: too many Gram work items");
   I.n_items = items;
@@ -651,8 +715,14 @@ int memi_ctf_distance(const void* plan_dev, const memi_plan_info* info, const vo
   // K steps per segment; a half spans two segments, split into chunks of spc steps (the last
   // one may be shorter)
   const int64_t steps = Khp / kstep;
-  const int64_t spc = (2 * steps + chunks - 1) / chunks;
-  MEMI_CHECK_ARG(steps < (1LL << 29) && (int64_t)(chunks - 1) * spc < 2 * steps,
+  int64_t spc = (2 * steps + chunks - 1) / chunks;
+  int live = chunks;                        // chunks that hold steps
+  if (info->auto_split) {
+    // short operands leave some of the plan's chunks empty; a chain stays within a segment
+    spc = std::min<int64_t>(std::max<int64_t>(spc, kAutoMinSteps), steps);
+    live = (int)((2 * steps + spc - 1) / spc);
+  }
+  MEMI_CHECK_ARG(steps < (1LL << 29) && (int64_t)(live - 1) * spc < 2 * steps && live <= chunks,
                  "memi_ctf_distance: %d chunks leave an empty chunk of the %lld K steps",
                  chunks, (long long)(2 * steps));
   MEMI_CHECK_ARG(kappa > 0, "memi_ctf_distance: kappa must be positive");
@@ -664,19 +734,18 @@ int memi_ctf_distance(const void* plan_dev, const memi_plan_info* info, const vo
   const int32_t* ut = (const int32_t*)(plan + info->off_utiles);
   const int64_t grid = ((info->n_items + 7) / 8) * 8;
   MEMI_CHECK_ARG(grid < (int64_t)1 << 31, "memi_ctf_distance: too many work items");
-  hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, flag_count, (int64_t)1);
-  MEMI_CHECK_LAUNCH("k_zero_i32");
   if (ev_start && hipEventRecord((hipEvent_t)ev_start, s) != hipSuccess) {
     set_error("memi_ctf_distance: hipEventRecord failed");
     return MEMI_ELAUNCH;
   }
-  // default schedule: prefetch two K steps for 128-wide tiles, one for 256-wide
-  const int depth = variant == 0 ? (BT == 128 ? 2 : 1) : variant;
+  // default schedule: straight into LDS (136 tiles of 128, N = 128, split-BF16, 12 chunks: 0.432
+  // ms, against 0.485 with a prefetch of two K steps through registers)
+  const int depth = variant == 0 ? 3 : variant;
   const char* lo = precision == MEMI_PREC_FP32 ? nullptr : (const char*)op_lo;
 #define MEMI_LAUNCH_GRAM(P, SH, V)                                                            \
   hipLaunchKernelGGL((k_gram_tiles<P, SH, V>), dim3((unsigned)grid), dim3(SH::NT), 0, s,       \
                      (const char*)op_hi, lo, Khp, (int)spc, (int)steps, items, info->n_items, \
-                     pds, ws)
+                     pds, ws, flag_count)
   if (precision == MEMI_PREC_FP32) {
     if (BT == 256 && depth == 3) MEMI_LAUNCH_GRAM(MEMI_PREC_FP32, Shape256, 3);
     else if (BT == 256) MEMI_LAUNCH_GRAM(MEMI_PREC_FP32, Shape256, 1);
@@ -696,9 +765,9 @@ int memi_ctf_distance(const void* plan_dev, const memi_plan_info* info, const vo
     set_error("memi_ctf_distance: hipEventRecord failed");
     return MEMI_ELAUNCH;
   }
-  hipLaunchKernelGGL(k_gram_finalize, dim3((unsigned)info->n_utiles, BT * BT / TB_FIN),
-                     dim3(256), 0, s, ut, pds, ws, chunks, BT, kappa, D, flags, info->flag_cap,
-                     flag_count);
+  hipLaunchKernelGGL(k_gram_finalize, dim3((unsigned)info->n_utiles, (BT / FB) * (BT / FB)),
+                     dim3(256), 0, s, ut, pds, ws, chunks, live, BT, kappa, D, flags,
+                     info->flag_cap, flag_count);
   MEMI_CHECK_LAUNCH("k_gram_finalize");
   hipLaunchKernelGGL(k_gram_recompute, dim3(1024), dim3(256), 0, s, flags, flag_count,
                      info->flag_cap, pds, (const float2*)fy, ctf_half, N, D);

@@ -133,6 +133,26 @@ def test_distance_rejects_a_split_with_an_empty_chunk():
     assert autotune.valid_chunks(nat.PREC_SPLIT_BF16, 8320, 3)
 
 
+@pytest.mark.parametrize("ns", [[1], [100], [900], [2000], [300] * 200])
+@pytest.mark.parametrize("tile", [128, 256])
+def test_plan_automatic_split(ns, tile):
+    """chunks <= 0 leaves the K split to the plan: at least two chunks (or the count asked for),
+    at most 64, tables and workspace for that count; counts outside -64..64 are refused."""
+    from manifoldem_python_amd import _native as nat
+    rows0 = np.concatenate(([0], np.cumsum(ns)[:-1]))
+    for least in (0, 6, 64):
+        pl = nat.Plan(rows0, ns, ns, chunks=-least, device="cpu", gram_tile=tile)
+        I = pl.info
+        assert I.auto_split == 1 and max(2, least) <= I.chunks <= 64
+        same = nat.Plan(rows0, ns, ns, chunks=I.chunks, device="cpu", gram_tile=tile)
+        assert same.info.auto_split == 0
+        assert (I.n_items, I.ws_floats) == (same.info.n_items, same.info.ws_floats)
+        np.testing.assert_array_equal(pl.host, same.host)
+    for bad in (-65, 65):
+        with pytest.raises(RuntimeError, match="npd/chunks"):
+            nat.Plan(rows0, ns, ns, chunks=bad, device="cpu", gram_tile=tile)
+
+
 def test_ritz_vectors_checks_meta_on_the_host():
     """A Ritz assembly whose basis length J exceeds the PD size (or k exceeds kmax) is refused
     before launch: the kernel indexes the basis and S by these numbers."""

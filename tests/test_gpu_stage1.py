@@ -238,6 +238,27 @@ def test_gram_uneven_chunks_vs_float64(cuda, precision, chunks, tile):
     assert np.all(np.diag(D) == 0)
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n,N,tile", [(2, 16, 128), (31, 16, 128), (33, 24, 256), (127, 32, 128),
+                                      (130, 48, 128), (261, 32, 256), (390, 24, 128)])
+def test_gram_automatic_split(cuda, precision, n, N, tile):
+    """The automatic K split (operands so short that some of its chunks stay empty, PD sizes
+    around the tiles' and the finalize blocks' sides) against two chunks: the same products in
+    sums cut elsewhere, so both are within the error model's 1e-5 of the exact distance and
+    within 2e-5 of each other; whole mirror, zero diagonal."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    s = _setup(n, N, seed=n)
+    geo, out, op = _gpu_prep(s, cuda, precision)
+    plan = nat.Plan([0], [n], [n], chunks=pl.CHUNKS[precision], gram_tile=tile)
+    assert plan.info.auto_split and plan.info.chunks >= 2
+    D = pl.ctf_distances(plan, op, out["fy"], out["ctf"], N).block(0).cpu().numpy()
+    two = nat.Plan([0], [n], [n], chunks=2, gram_tile=tile)
+    D2 = pl.ctf_distances(two, op, out["fy"], out["ctf"], N).block(0).cpu().numpy()
+    assert rel_offdiag(D, D2).max() < 2e-5
+    np.testing.assert_array_equal(D, D.T)
+    assert np.all(np.diag(D) == 0)
+
+
 def _operand_values(op):
     import torch
     if op.lo is None:
