@@ -39,82 +39,168 @@ __global__ __launch_bounds__(256) void k_condist(const T* __restrict__ D,
 
 // ------------------------------------------------------------ supervector spectra -------
 // out[ii][c][k] = sum_{i<m} mu_psi[i][c] * spec[j][k] C[j][k] / W_i[k], j = C-1-ii+i,
-// W_i[k] = sum_{t=i+1}^{i+C} C[t][k]^2 + 1/snr.  Thread = (frequency k, group of G delays);
-// the G spectra a thread needs slide by one image per step, so they live in a register ring.
-constexpr int SG = 5;
+// W_i[k] = sum_{t=i+1}^{i+C} C[t][k]^2 + 1/snr.
+//
+// A wave takes SG delays and four of the ell weights of 64 frequencies: 8 SG float32 sums per
+// lane.  The waves of a workgroup hold the other delays and weights of the same frequencies and
+// share the weights u[i][c] = mu_psi[i][c] / W_i (float64, rounded once), which they compute in
+// turn, SG steps ahead, into LDS.  The spectra slide by one image per step; SG steps are unrolled
+// so that every G sits in a register of its own.  With few frequencies a wave takes 2^kshift of
+// them and cuts the steps into 64 >> kshift pieces, summed across its lanes at the end.
+//
+// Bound: float32 multiply-add issue (8 SG per step against ~25 other instructions) at two waves
+// per SIMD, and 203 workgroups on 256 CUs: 1500 images of 160 x 160, 50 delays, 8 weights take
+// 0.75 ms (40 TFLOP/s); 1.63 ms with 5 delays x 8 weights per thread, where each thread formed
+// its own eight weights with a float64 division every 80 sums and waited for each step's loads.
 constexpr int ELLMAX = 8;
 
-__global__ __launch_bounds__(256) void k_supervectors(const float2* __restrict__ spec,
-                                                      const float* __restrict__ ctf, int n,
-                                                      int64_t Kh, int C,
-                                                      const double* __restrict__ mu_psi, int ell,
-                                                      double snr, float2* __restrict__ out) {
-  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int g0 = blockIdx.y * SG;
-  if (k >= Kh) return;
+template <int SG, typename OFF>
+__global__ __launch_bounds__(512) void k_supervectors(
+    const float2* __restrict__ spec, const float* __restrict__ ctf, int n, int64_t Kh, int C,
+    const double* __restrict__ mu_psi, int ell, double snr, int kshift, int steps, int gpb,
+    int halves, float2* __restrict__ out) {
+  __shared__ float4 us[2][SG][2][64];        // the weights of two rounds of SG steps
+  __shared__ double ws[SG][64];
+  __shared__ double mus[2][SG * ELLMAX * 16];  // mu_psi of two rounds: [step][c][piece]
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  const int half = w % halves;
+  const int g0 = ((int)blockIdx.y * gpb + w / halves) * SG;     // this wave's first delay
+  const int64_t k = ((int64_t)blockIdx.x << kshift) + (lane & ((1 << kshift) - 1));
+  const int64_t kc = min(k, Kh - 1);
   const int m = n - C;
-  // W_0 = sum_{t=1}^{C} C_t^2
+  const int i0 = (lane >> kshift) * steps;                       // this lane's steps
+  // element offsets (OFF: 32 bits when they fit, one register per address); images outside the
+  // steps' range are read at its ends and weigh zero
+  auto img = [&](int j) { return (OFF)min(max(j, 0), n - 2) * (OFF)Kh + (OFF)kc; };
+  auto ctf_at = [&](int t) { return ctf[(OFF)min(t, n - 1) * (OFF)Kh + (OFF)kc]; };
   double W = 1.0 / snr;
   for (int t = 1; t <= C; ++t) {
-    const double c = ctf[(int64_t)t * Kh + k];
+    const double c = ctf_at(i0 + t);
     W += c * c;
   }
-  float2 ring[SG];
-  const int jmax0 = C - 1 - g0;
-#pragma unroll
-  for (int t = 0; t < SG; ++t) {
-    // ring[SG-1-t] holds G_{jmax - t}; preload all but the newest (t = 0)
-    const int j = jmax0 - t;
-    float2 g = make_float2(0.f, 0.f);
-    if (t > 0 && j >= 0 && g0 + t < C) {
-      const float2 x = spec[(int64_t)j * Kh + k];
-      const float c = ctf[(int64_t)j * Kh + k];
-      g = make_float2(x.x * c, x.y * c);
+  // mu_psi of steps c0 .. c0 + SG - 1 into LDS, zero past a piece's end
+  const int pieces = 64 >> kshift;
+  auto stage_mu = [&](int c0, double* to) {
+#pragma unroll 1
+    for (int e = threadIdx.x; e < SG * ell * pieces; e += blockDim.x) {
+      const int q = e / (SG * ell), r = e % (SG * ell);
+      const int st = c0 + r / ell, i = q * steps + st;
+      to[r * pieces + q] = (st < steps && i < m) ? mu_psi[(int64_t)i * ell + r % ell] : 0.0;
     }
-    ring[SG - 1 - t] = g;
-  }
-  float acc[SG][ELLMAX][2];
-#pragma unroll
-  for (int t = 0; t < SG; ++t)
-#pragma unroll
-    for (int c = 0; c < ELLMAX; ++c) acc[t][c][0] = acc[t][c][1] = 0.f;
-  for (int i = 0; i < m; ++i) {
-    const int jn = jmax0 + i;  // newest image needed at this step
-    {
-      const float2 x = spec[(int64_t)jn * Kh + k];
-      const float c = ctf[(int64_t)jn * Kh + k];
-      ring[SG - 1] = make_float2(x.x * c, x.y * c);
-    }
-    const double invW = 1.0 / W;
-    float u[ELLMAX];
-#pragma unroll
-    for (int c = 0; c < ELLMAX; ++c) u[c] = (c < ell) ? (float)(mu_psi[(int64_t)i * ell + c] * invW) : 0.f;
+  };
+  // the CTFs that leave and enter the window over steps c0 .. c0 + SG - 1
+  float wa[SG], wb[SG];
+  auto window = [&](int c0) {
 #pragma unroll
     for (int t = 0; t < SG; ++t) {
-      const float2 g = ring[SG - 1 - t];
-#pragma unroll
-      for (int c = 0; c < ELLMAX; ++c) {
-        acc[t][c][0] += u[c] * g.x;
-        acc[t][c][1] += u[c] * g.y;
-      }
+      wa[t] = ctf_at(i0 + c0 + t + 1);
+      wb[t] = ctf_at(i0 + c0 + t + 1 + C);
     }
-    // slide: drop the oldest, W_{i+1} = W_i - C_{i+1}^2 + C_{i+1+C}^2
+  };
+  // The weights of those steps: wave w computes every nw-th of them.  Every wave runs the window
+  // sum through all steps and keeps its own ones in LDS (nobody else reads them), so that the
+  // divisions stay out of the unrolled code, where they cost registers.
+  auto weights = [&](float4(*u)[2][64], const double* mu) {
 #pragma unroll
-    for (int t = 0; t < SG - 1; ++t) ring[t] = ring[t + 1];
-    if (i + 1 < m) {
-      const double a = ctf[(int64_t)(i + 1) * Kh + k];
-      const double b = ctf[(int64_t)(i + 1 + C) * Kh + k];
+    for (int t = 0; t < SG; ++t) {
+      if (t % nw == w) ws[t][lane] = W;
+      const double a = wa[t], b = wb[t];
       W += b * b - a * a;
     }
-  }
+#pragma unroll 1
+    for (int t = w; t < SG; t += nw) {
+      const double invW = 1.0 / ws[t][lane];
+      const double* mp = mu + t * ell * pieces + (lane >> kshift);
+#pragma unroll 1
+      for (int h = 0; h < halves; ++h) {
+        float v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          v[c] = 4 * h + c < ell ? (float)(mp[(4 * h + c) * pieces] * invW) : 0.f;
+        u[t][h][lane] = make_float4(v[0], v[1], v[2], v[3]);
+      }
+    }
+  };
+  float2 prev[SG], cur[SG], nx[SG];
+  float nc[SG];
+  const int j0 = C - 1 - g0 + i0;            // newest image of delay g0 at the first step
 #pragma unroll
   for (int t = 0; t < SG; ++t) {
-    const int ii = g0 + t;
-    if (ii >= C) break;
-#pragma unroll
-    for (int c = 0; c < ELLMAX; ++c)       // constant indices keep acc in registers
-      if (c < ell) out[((int64_t)ii * ell + c) * Kh + k] = make_float2(acc[t][c][0], acc[t][c][1]);
+    const OFF a = img(j0 - SG + t), b = img(j0 + t);
+    const float2 x = spec[a], y = spec[b];
+    const float cx = ctf[a], cy = ctf[b];
+    prev[t] = make_float2(x.x * cx, x.y * cx);
+    cur[t] = make_float2(y.x * cy, y.y * cy);
   }
+  float acc[SG][4][2];
+#pragma unroll
+  for (int d = 0; d < SG; ++d)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[d][c][0] = acc[d][c][1] = 0.f;
+  stage_mu(0, mus[0]);
+  stage_mu(SG, mus[1]);
+  window(0);
+  __syncthreads();
+  weights(us[0], mus[0]);
+  int b = 0;
+  for (int c0 = 0; c0 < steps; c0 += SG) {
+    __syncthreads();       // this round's weights are in us[b], the next one's mu in mus[b ^ 1]
+    stage_mu(c0 + 2 * SG, mus[b]);
+    if (g0 >= C) window(c0 + SG);            // a wave with no delays left only computes weights
+    else {
+#pragma unroll
+      for (int t = 0; t < SG; ++t) {
+        const OFF a = img(j0 + c0 + SG + t);
+        nx[t] = spec[a];
+        nc[t] = ctf[a];
+      }
+      float4 un = us[b][0][half][lane];
+#pragma unroll
+      for (int t = 0; t < SG; ++t) {
+        const float4 u = un;
+        if (t + 1 < SG) un = us[b][t + 1][half][lane];
+#pragma unroll
+        for (int d = 0; d < SG; ++d) {
+          const float2 g = t >= d ? cur[t >= d ? t - d : 0] : prev[t >= d ? 0 : SG + t - d];
+          acc[d][0][0] += u.x * g.x;
+          acc[d][0][1] += u.x * g.y;
+          acc[d][1][0] += u.y * g.x;
+          acc[d][1][1] += u.y * g.y;
+          acc[d][2][0] += u.z * g.x;
+          acc[d][2][1] += u.z * g.y;
+          acc[d][3][0] += u.w * g.x;
+          acc[d][3][1] += u.w * g.y;
+        }
+        // loads in flight across the second half, whose history needs fewer registers
+        if (t == SG / 2) window(c0 + SG);
+      }
+#pragma unroll
+      for (int t = 0; t < SG; ++t) {
+        prev[t] = cur[t];
+        cur[t] = make_float2(nx[t].x * nc[t], nx[t].y * nc[t]);
+      }
+    }
+    b ^= 1;
+    if (c0 + SG < steps) weights(us[b], mus[b]);
+  }
+  for (int off = 1 << kshift; off < 64; off <<= 1)
+#pragma unroll
+    for (int d = 0; d < SG; ++d)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        acc[d][c][0] += __shfl_xor(acc[d][c][0], off, 64);
+        acc[d][c][1] += __shfl_xor(acc[d][c][1], off, 64);
+      }
+  if ((lane >> kshift) != 0 || k >= Kh) return;
+#pragma unroll
+  for (int d = 0; d < SG; ++d)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (g0 + d < C && 4 * half + c < ell)
+        out[((int64_t)(g0 + d) * ell + 4 * half + c) * Kh + k] =
+            make_float2(acc[d][c][0], acc[d][c][1]);
 }
 
 // ------------------------------------------------------------- tall-skinny algebra -------
@@ -581,9 +667,53 @@ int memi_nlsa_supervectors(const void* spec, const float* ctf_half, int n, int N
   MEMI_CHECK_ARG(con_order >= 1 && n > con_order && snr > 0,
                  "memi_nlsa_supervectors: bad n=%d ConOrder=%d", n, con_order);
   const int64_t Kh = (int64_t)N * (N / 2 + 1);
-  dim3 g((unsigned)((Kh + 255) / 256), (unsigned)((con_order + SG - 1) / SG));
-  hipLaunchKernelGGL(k_supervectors, g, dim3(256), 0, (hipStream_t)stream, (const float2*)spec,
-                     ctf_half, n, Kh, con_order, mu_psi, ell, snr, (float2*)out);
+  // Delays per wave (9 to 13), and pieces of the steps per wave.  A CU runs eight waves; a step
+  // of a workgroup takes its waves per SIMD times 8 sg sums and ~25 other instructions, and each
+  // piece starts with its own window sum (C loads) and history.
+  const int halves = (ell + 3) / 4;
+  const int m = n - con_order;
+  int sg = 0, gy = 0, gpb = 0, kshift = 6;
+  double best = 0.0;
+  for (int g = 13; g >= 9; --g) {
+    const int groups = (con_order + g - 1) / g;
+    const int y = (groups * halves + 7) / 8;
+    const int per = (groups + y - 1) / y;          // delay groups per workgroup: <= 8 waves
+    const int64_t res = 256 * (8 / (per * halves));
+    for (int ks = 6; ks >= 2; --ks) {
+      const int64_t blocks = ((Kh + (1 << ks) - 1) >> ks) * y;
+      const double cost = (double)((blocks + res - 1) / res) * (8 / (per * halves)) *
+                          ((per * halves + 3) / 4) * (8 * g + 25) *
+                          ((double)m / (64 >> ks) + 0.5 * con_order + 2 * g);
+      if (sg == 0 || cost < best) {
+        best = cost;
+        sg = g;
+        gy = y;
+        gpb = per;
+        kshift = ks;
+      }
+    }
+  }
+  const int pieces = 64 >> kshift;
+  const int steps = (m + pieces - 1) / pieces;
+  const int64_t gx = (Kh + (1 << kshift) - 1) >> kshift;
+  MEMI_CHECK_ARG(gx < 0x7fffffffLL && gy < 65536, "memi_nlsa_supervectors: too large");
+  const dim3 grid((unsigned)gx, (unsigned)gy), block(64 * gpb * halves);
+  const bool small = (int64_t)n * Kh < (1LL << 29);      // byte offsets within 32 bits
+#define MEMI_SUPERVECTORS(G)                                                                    \
+  do {                                                                                          \
+    auto kern = small ? k_supervectors<G, uint32_t> : k_supervectors<G, int64_t>;               \
+    hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, (const float2*)spec, ctf_half, \
+                       n, Kh, con_order, mu_psi, ell, snr, kshift, steps, gpb, halves,          \
+                       (float2*)out);                                                           \
+  } while (0)
+  switch (sg) {
+    case 9: MEMI_SUPERVECTORS(9); break;
+    case 10: MEMI_SUPERVECTORS(10); break;
+    case 11: MEMI_SUPERVECTORS(11); break;
+    case 12: MEMI_SUPERVECTORS(12); break;
+    default: MEMI_SUPERVECTORS(13); break;
+  }
+#undef MEMI_SUPERVECTORS
   MEMI_CHECK_LAUNCH("k_supervectors");
   return MEMI_OK;
 }

@@ -66,6 +66,34 @@ def test_supervectors_match_fft_loop(cuda, pd_case):
     assert err < 2e-6, err
 
 
+@pytest.mark.parametrize("n,N,C,ell", [(2, 8, 1, 1), (40, 9, 9, 4), (61, 16, 14, 5), (130, 12, 27, 8),
+                                       (200, 33, 50, 3), (97, 20, 60, 8), (150, 96, 20, 8),
+                                       (120, 11, 97, 2)])
+def test_supervector_spectra_tiles(cuda, n, N, C, ell):
+    """Delays and weights around the kernel's tiles (1, one wave's 9 to 13, several workgroups of
+    them; 1 to 8 weights), few and many frequencies (steps cut into 1 to 16 pieces, also more
+    pieces than steps), against the float64 sum.  A float32 sum of m products of rounded factors
+    is within (m + 3) 2^-24 of the sum of their magnitudes."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(n)
+    Kh, m = N * (N // 2 + 1), n - C
+    spec = (rng.normal(size=(n, Kh)) + 1j * rng.normal(size=(n, Kh))).astype(np.complex64)
+    ctf = rng.uniform(-1, 1, (n, Kh)).astype(np.float32)
+    mu = rng.normal(size=(m, ell))
+    sv = torch.full((C, ell, Kh), np.nan, dtype=torch.complex64, device=cuda)
+    nat.nlsa_supervectors(torch.as_tensor(spec, device=cuda), torch.as_tensor(ctf, device=cuda), n,
+                          N, C, torch.as_tensor(mu, device=cuda), 5.0, sv)
+    got = sv.cpu().numpy()
+    c2 = ctf.astype(np.float64) ** 2
+    W = np.stack([c2[i + 1:i + 1 + C].sum(0) for i in range(m)]) + 1.0 / 5
+    G = spec.astype(np.complex128) * ctf
+    for ii in range(C):
+        g = G[C - 1 - ii:C - 1 - ii + m] / W
+        ref, mag = mu.T @ g, np.abs(mu).T @ (np.abs(g.real) + np.abs(g.imag))
+        assert np.all(np.abs(got[ii] - ref) <= (m + 3) * 2.0 ** -24 * mag), ii
+
+
 def test_nlsa_matches_oracle(cuda, pd_case):
     import torch
     from manifoldem_python_amd import spectral, fit1d
