@@ -267,6 +267,7 @@ __global__ void k_col_sum(const double* __restrict__ U, int64_t npix, int q,
   const int col = blockIdx.y * blockDim.x + threadIdx.x;
   if (col >= q) return;
   double s = 0.0;
+#pragma unroll 8
   for (int64_t p = blockIdx.x; p < npix; p += gridDim.x) s += U[p * q + col];
   atomicAdd(&colsum[col], s);
 }
@@ -279,83 +280,147 @@ __global__ void k_col_center(double* __restrict__ U, int64_t npix, int q,
     U[e] -= colsum[e % q] / (double)npix;
 }
 
-// G[a][b] += sum_p U[p][a] U[p][b] over this block's pixel range; 16x16 tiles of G
+// G[a][b] += sum_p U[p][a] U[p][b] over a wave's pixel range, on v_mfma_f64_16x16x4_f64: one 16x16
+// tile (a0 <= b0) of G per wave, four pixels per instruction straight from memory (a lane reads
+// U[p + l / 16][a0 + l % 16], whole 128-byte lines), eight instructions' loads in flight.  Every
+// tile below the diagonal is its mirror's transpose.  Bound: memory latency (npix = 25600,
+// q = 100: 32 us; 100 us with both operands through LDS on the vector units).
+typedef double doublex4_t __attribute__((ext_vector_type(4)));
+constexpr int GC_ROWS = 512;               // pixels per wave
+
 __global__ __launch_bounds__(256) void k_gram_cols(const double* __restrict__ U, int64_t npix,
-                                                   int q, int64_t pchunk, double* __restrict__ G) {
-  __shared__ double ta[64][17], tb[64][17];
+                                                   int q, double* __restrict__ G) {
+  if (blockIdx.y < blockIdx.x) return;
   const int a0 = blockIdx.x * 16, b0 = blockIdx.y * 16;
-  const int ta_i = threadIdx.x & 15, tb_i = threadIdx.x >> 4;
-  const int64_t p0 = blockIdx.z * pchunk, p1 = min(npix, p0 + pchunk);
-  double s = 0.0;
-  for (int64_t pb = p0; pb < p1; pb += 64) {
-    for (int e = threadIdx.x; e < 64 * 16; e += blockDim.x) {
-      const int r = e / 16, cc = e % 16;
-      const int64_t p = pb + r;
-      ta[r][cc] = (p < p1 && a0 + cc < q) ? U[p * q + a0 + cc] : 0.0;
-      tb[r][cc] = (p < p1 && b0 + cc < q) ? U[p * q + b0 + cc] : 0.0;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int64_t p0 = ((int64_t)blockIdx.z * 4 + (threadIdx.x >> 6)) * GC_ROWS;
+  const int64_t p1 = min(npix, p0 + GC_ROWS);
+  const bool ina = a0 + lr < q, inb = b0 + lr < q;
+  const double* ua = U + (ina ? a0 + lr : 0);
+  const double* ub = U + (inb ? b0 + lr : 0);
+  doublex4_t acc = {};
+  for (int64_t pb = p0; pb < p1; pb += 32) {
+    double a[8], b[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int64_t p = pb + 4 * e + lk;
+      const bool in = p < p1;
+      const int64_t at = (in ? p : p0) * q;
+      a[e] = in && ina ? ua[at] : 0.0;
+      b[e] = in && inb ? ub[at] : 0.0;
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int r = 0; r < 64; ++r) s += ta[r][ta_i] * tb[r][tb_i];
-    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[e], b[e], acc, 0, 0, 0);
   }
-  const int a = a0 + ta_i, b = b0 + tb_i;
-  if (a < q && b < q) atomicAdd(&G[a * q + b], s);
+  if (p0 >= npix || !inb) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int i = a0 + lk + 4 * e, j = b0 + lr;
+    if (i >= q) continue;
+    atomicAdd(&G[i * q + j], acc[e]);
+    if (a0 != b0) atomicAdd(&G[j * q + i], acc[e]);
+  }
 }
 
-// IMGT[p][j] = inv_sd[j] * sum_q Ubar[p][q] H[q][j]   (float64, 64x64 tiles, 4x4 per thread)
-__global__ __launch_bounds__(256) void k_imgt(const double* __restrict__ U,
-                                              const double* __restrict__ H,
-                                              const double* __restrict__ inv_sd, int64_t npix,
-                                              int q, int ncols, double* __restrict__ out) {
-  __shared__ double us[16][65], hs[16][65];
-  const int64_t p0 = (int64_t)blockIdx.y * 64;
-  const int j0 = blockIdx.x * 64;
-  const int tr = threadIdx.x >> 4, tc = threadIdx.x & 15;
-  double acc[4][4] = {};
-  for (int k0 = 0; k0 < q; k0 += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += blockDim.x) {
-      const int kk = e / 64, x = e % 64;
-      const int64_t p = p0 + x;
-      us[kk][x] = (p < npix && k0 + kk < q) ? U[p * q + k0 + kk] : 0.0;
-      hs[kk][x] = (j0 + x < ncols && k0 + kk < q) ? H[(int64_t)(k0 + kk) * ncols + j0 + x] : 0.0;
+// IMGT[p][j] = inv_sd[j] * sum_q Ubar[p][q] H[q][j] on v_mfma_f64_16x16x4_f64: 64 x 128 outputs
+// per workgroup, 32 x 64 per wave (8 blocks of 16 x 16), K in pieces of 20 through LDS.  Lane l
+// of an MFMA holds A[l % 16][l / 16], B[l / 16][l % 16] and rows l / 16 + 4 r of column l % 16 of
+// the result.
+//
+// Bound: the float64 MFMAs and writing IMGT (npix = 25600, q = 100, 1400 columns: 98 us at the
+// rate a large float64 product reaches, 58 us at a large copy's): 227 us, with the next piece's
+// loads in flight during the products and two workgroups per CU (three without the prefetch: 280
+// us; 128 x 128 outputs, one workgroup per CU: 454; the vector units with 4 x 4 outputs per
+// thread, two LDS reads for every two products: 410).
+constexpr int IM_P = 64, IM_J = 128, IM_K = 20;
+typedef double doublex4_t __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256, 2) void k_imgt(const double* __restrict__ U,
+                                                 const double* __restrict__ H,
+                                                 const double* __restrict__ inv_sd, int64_t npix,
+                                                 int q, int ncols, double* __restrict__ out) {
+  __shared__ double us2[2][IM_K][IM_P + 2], hs2[2][IM_K][IM_J + 2];
+  const int64_t p0 = (int64_t)blockIdx.y * IM_P;
+  const int j0 = blockIdx.x * IM_J;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int pw = (wv >> 1) * 32, jw = (wv & 1) * 64;            // this wave's corner
+  const int lr = lane & 15, lk = lane >> 4;
+  doublex4_t acc[2][4] = {};
+  constexpr int NU = IM_P * IM_K / 256, NH = IM_J * IM_K / 256;
+  double ru[NU], rh[NH];                     // the next piece, loaded during this one's products
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int e = 0; e < NU; ++e) {
+      const int f = threadIdx.x + 256 * e, pr = f / IM_K, pk = k0 + f % IM_K;   // along U's rows
+      ru[e] = (p0 + pr < npix && pk < q) ? U[(p0 + pr) * q + pk] : 0.0;
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      double a[4], b[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        a[x] = us[kk][tr * 4 + x];
-        b[x] = hs[kk][tc * 4 + x];
-      }
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) acc[x][y] += a[x] * b[y];
+    for (int e = 0; e < NH; ++e) {
+      const int f = threadIdx.x + 256 * e, hk = k0 + f / IM_J, hj = j0 + f % IM_J;  // along H's
+      rh[e] = (hj < ncols && hk < q) ? H[(int64_t)hk * ncols + hj] : 0.0;
     }
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int e = 0; e < NU; ++e) {
+      const int f = threadIdx.x + 256 * e;
+      us2[b][f % IM_K][f / IM_K] = ru[e];
+    }
+#pragma unroll
+    for (int e = 0; e < NH; ++e) {
+      const int f = threadIdx.x + 256 * e;
+      hs2[b][f / IM_J][f % IM_J] = rh[e];
+    }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  int bf = 0;
+  for (int k0 = 0; k0 < q; k0 += IM_K, bf ^= 1) {
+    double(*us)[IM_P + 2] = us2[bf];
+    double(*hs)[IM_J + 2] = hs2[bf];
+    load(k0 + IM_K);
+#pragma unroll
+    for (int k = 0; k < IM_K; k += 4) {
+      double a[2], b[4];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) a[r] = us[k + lk][pw + 16 * r + lr];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) b[c] = hs[k + lk][jw + 16 * c + lr];
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[c], acc[r][c], 0, 0, 0);
+    }
+    store(bf ^ 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    const int64_t p = p0 + tr * 4 + x;
-    if (p >= npix) continue;
+  for (int c = 0; c < 4; ++c) {
+    const int j = j0 + jw + 16 * c + lr;
+    if (j >= ncols) continue;
+    const double sd = inv_sd[j];
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
-      const int j = j0 + tc * 4 + y;
-      if (j < ncols) out[p * ncols + j] = acc[x][y] * inv_sd[j];
-    }
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t p = p0 + pw + 16 * r + lk + 4 * e;
+        if (p < npix) out[p * ncols + j] = acc[r][c][e] * sd;
+      }
   }
 }
 
 // ---------------------------------------------------------- reconstruction distances ----
-// T[a][j] = sum_b Gq[a][b] H[b][j]   (Gq [q][q], H [q][ncols])
+// T[a][j] = sum_b Gq[a][b] H[b][j]   (Gq [q][q], H [q][ncols]).  One output per thread; eight
+// terms' loads go out together (one at a time: 41 us instead of 11 for q = 100, 1400 columns).
 __global__ void k_gq_h(const double* __restrict__ Gq, const double* __restrict__ H, int q,
                        int ncols, double* __restrict__ T) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const int a = blockIdx.y;
   if (j >= ncols) return;
   double s = 0.0;
+#pragma unroll 8
   for (int b = 0; b < q; ++b) s = fma(Gq[a * q + b], H[(int64_t)b * ncols + j], s);
   T[(int64_t)a * ncols + j] = s;
 }
@@ -368,6 +433,7 @@ __global__ void k_recon_diag(const double* __restrict__ H, const double* __restr
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= ncols) return;
   double s = 0.0;
+#pragma unroll 8
   for (int a = 0; a < q; ++a) s = fma(H[(int64_t)a * ncols + j], T[(int64_t)a * ncols + j], s);
   dg[j] = s;
   inv_sd[j] = 1.0 / sqrt(s / npix);
@@ -756,10 +822,9 @@ int memi_center_gram(double* U2, int64_t npix, int q_dim, double* G, void* strea
   MEMI_CHECK_LAUNCH("k_col_center");
   hipLaunchKernelGGL(k_zero_d, dim3(1), dim3(256), 0, s, G, (int64_t)q_dim);
   MEMI_CHECK_LAUNCH("k_zero_d");
-  const int64_t pchunk = 1024;
   dim3 gg((unsigned)((q_dim + 15) / 16), (unsigned)((q_dim + 15) / 16),
-          (unsigned)((npix + pchunk - 1) / pchunk));
-  hipLaunchKernelGGL(k_gram_cols, gg, dim3(256), 0, s, U2, npix, q_dim, pchunk, G);
+          (unsigned)((npix + 4 * GC_ROWS - 1) / (4 * GC_ROWS)));
+  hipLaunchKernelGGL(k_gram_cols, gg, dim3(256), 0, s, U2, npix, q_dim, G);
   MEMI_CHECK_LAUNCH("k_gram_cols");
   return MEMI_OK;
 }
@@ -768,7 +833,7 @@ int memi_nlsa_imgt(const double* Ubar, const double* H, const double* inv_sd, in
                    int q_dim, int ncols, double* IMGT, void* stream) {
   MEMI_CHECK_ARG(Ubar && H && inv_sd && IMGT && npix > 0 && q_dim > 0 && ncols > 0,
                  "memi_nlsa_imgt: bad arguments");
-  dim3 g((unsigned)((ncols + 63) / 64), (unsigned)((npix + 63) / 64));
+  dim3 g((unsigned)((ncols + IM_J - 1) / IM_J), (unsigned)((npix + IM_P - 1) / IM_P));
   hipLaunchKernelGGL(k_imgt, g, dim3(256), 0, (hipStream_t)stream, Ubar, H, inv_sd, npix, q_dim,
                      ncols, IMGT);
   MEMI_CHECK_LAUNCH("k_imgt");

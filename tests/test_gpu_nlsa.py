@@ -94,6 +94,34 @@ def test_supervector_spectra_tiles(cuda, n, N, C, ell):
         assert np.all(np.abs(got[ii] - ref) <= (m + 3) * 2.0 ** -24 * mag), ii
 
 
+@pytest.mark.parametrize("npix,q,ncols", [(1, 1, 1), (64, 2, 127), (129, 19, 128), (600, 20, 130),
+                                          (2050, 41, 257), (127, 100, 15), (5000, 33, 40)])
+def test_frame_products_on_tiles(cuda, npix, q, ncols):
+    """The float64 matrix-core products of the reconstruction at the edges of their tiles (16 and
+    128 outputs, 20 of the contraction, 512 pixels per wave): the centred Gram of the columns and
+    the frames, against numpy.  A float64 sum of n products in any order is within n 2^-53 of the
+    sum of their magnitudes; two such roundings (numpy's and the kernel's), and the centring's."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(npix + q)
+    U = rng.normal(size=(npix, q))
+    H, sd = rng.normal(size=(q, ncols)), rng.uniform(0.5, 2, ncols)
+    Ud = torch.as_tensor(U, device=cuda)
+    G = torch.full((q, q), np.nan, dtype=torch.float64, device=cuda)
+    nat.center_gram(Ud, G)
+    Uc = U - U.mean(axis=0)
+    eps = 2.0 ** -53
+    scale = np.abs(U).sum(axis=0) + 1.0
+    np.testing.assert_allclose(Ud.cpu().numpy(), Uc, rtol=0, atol=8 * eps * scale.max())
+    Uc = Ud.cpu().numpy()
+    mag = np.abs(Uc).T @ np.abs(Uc)
+    assert np.all(np.abs(G.cpu().numpy() - Uc.T @ Uc) <= 2 * (npix + 2) * eps * mag)
+    out = torch.full((npix, ncols), np.nan, dtype=torch.float64, device=cuda)
+    nat.nlsa_imgt(Ud, torch.as_tensor(H, device=cuda), torch.as_tensor(sd, device=cuda), out)
+    ref, mag = (Uc @ H) * sd, (np.abs(Uc) @ np.abs(H)) * sd
+    assert np.all(np.abs(out.cpu().numpy() - ref) <= 2 * (q + 2) * eps * mag)
+
+
 def test_nlsa_matches_oracle(cuda, pd_case):
     import torch
     from manifoldem_python_amd import spectral, fit1d
