@@ -264,7 +264,10 @@ __global__ __launch_bounds__(256) void k_ferguson_thr(const int32_t* __restrict_
   }
 }
 
-// sweep: block = (256 eps values) x (one full tile); entries staged through LDS
+// sweep: block = (256 eps values) x (blockIdx.z-th part of one full tile); entries staged through
+// LDS.  Every thread walks its part's entries for its own eps, so the part's length is the
+// latency: the host cuts the tiles of small launches into up to 32 parts (one PD of 200, 101
+// eps: 1470 us with whole tiles, 56 us in 32 parts).
 __global__ __launch_bounds__(256) void k_ferguson_sweep(const int32_t* __restrict__ ftiles,
                                                         const memi_pd_desc* __restrict__ pds,
                                                         const float* __restrict__ D,
@@ -293,7 +296,9 @@ __global__ __launch_bounds__(256) void k_ferguson_sweep(const int32_t* __restric
   const double c = active ? 1.0 / (2.0 * exp(logEps[e_idx])) : 0.0;
   const double L2E = 1.4426950408889634;
   double S = 0.0, SX = 0.0, CN = 0.0;
-  for (int base = 0; base < TB * TB; base += SUB) {
+  const int part = TB * TB / gridDim.z;
+  const int p1 = (blockIdx.z + 1) * part;
+  for (int base = blockIdx.z * part; base < p1; base += SUB) {
     // stage this thread's 8 entries, compact the kernel entries
     float v8[SUB / 256];
     int cnt = 0;
@@ -302,7 +307,7 @@ __global__ __launch_bounds__(256) void k_ferguson_sweep(const int32_t* __restric
       const int e = base + threadIdx.x * (SUB / 256) + q;
       const int i = f[1] * TB + e / TB, j = f[2] * TB + e % TB;
       double v = -1.0;
-      if (i < P.n && j < P.n) v = entry_value(D, mask, P, W, full, i, j);
+      if (e < p1 && i < P.n && j < P.n) v = entry_value(D, mask, P, W, full, i, j);
       v8[q] = (float)v;
       cnt += (v >= 0);
     }
@@ -539,6 +544,12 @@ __global__ __launch_bounds__(256) void k_fer_moments(const int32_t* __restrict__
   const int b0 = (int)g[3], B = (int)g[4];
   if (B <= 0) return;                                 // uniform over the block
   for (int q = threadIdx.x; q < B * FM_NM; q += blockDim.x) ms[q] = 0.0;
+  // the bucket edges, behind the sums where the table leaves room (all but the widest grids): an
+  // entry then takes one log instead of a log and four exps
+  const bool tab = B * FM_NM + B + 1 <= FM_BMAX * FM_NM;
+  double* edge = ms + B * FM_NM;
+  if (tab)
+    for (int q = threadIdx.x; q <= B; q += blockDim.x) edge[q] = exp(base + (b0 + q) * w);
   const int W = (P.n + 31) / 32;
   const bool full = P.k >= P.n;
   __shared__ TileMaskT mt;
@@ -551,8 +562,19 @@ __global__ __launch_bounds__(256) void k_fer_moments(const int32_t* __restrict__
     if (i >= P.n || j >= P.n) continue;
     const double v = entry_value_t(D, mask, P, W, full, i, j, mt, il, jl);
     if (v <= 0.0) continue;
-    const int k = min(max(fm_bucket(v, base, w) - b0, 0), B - 1);
-    const double lo = exp(base + (b0 + k) * w), hi = exp(base + (b0 + k + 1) * w);
+    int k = (int)floor((log(v) - base) / w) - b0;
+    double lo, hi;
+    if (tab && k >= 0 && k < B) {
+      if (v < edge[k]) --k;
+      else if (v >= edge[k + 1]) ++k;
+      k = min(max(k, 0), B - 1);
+      lo = edge[k];
+      hi = edge[k + 1];
+    } else {
+      k = min(max(fm_bucket(v, base, w) - b0, 0), B - 1);
+      lo = exp(base + (b0 + k) * w);
+      hi = exp(base + (b0 + k + 1) * w);
+    }
     const double u = (v - 0.5 * (lo + hi)) / (0.5 * (hi - lo));
     double pw = 1.0;
     for (int m = 0; m < FM_NM; ++m) {
@@ -575,7 +597,11 @@ __global__ void k_fer_thr_copy(int64_t npd, const double* __restrict__ st,
   }
 }
 
-// one thread per eps: the series over the buckets below the eps's cut
+// FM_LANES threads per eps: the series over the buckets below the eps's cut, every FM_LANES-th of
+// them each (one thread per eps walks up to 544 dependent series: one PD of 1273, 1501 eps 73 us
+// with one, 10 us with eight)
+constexpr int FM_LANES = 8;
+
 __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restrict__ logEps,
                                                            int n_eps,
                                                            const double* __restrict__ gp,
@@ -593,9 +619,11 @@ __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restr
     hw[k] = 0.5 * (hi - lo);
   }
   __syncthreads();
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x % FM_LANES;
+  const int e = blockIdx.x * (blockDim.x / FM_LANES) + threadIdx.x / FM_LANES;
   if (e >= n_eps) return;
   if (g[7] != 0.0) {                  // direct-sweep PD: cleared for its accumulation
+    if (lane != 0) return;
     double* o = out + ((int64_t)pd * n_eps + e) * 3;
     o[0] = o[1] = o[2] = 0.0;
     return;
@@ -608,8 +636,8 @@ __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restr
   const double c = 1.0 / (2.0 * exp(logEps[e]));
   const int jmax = min(B, max(0, e * s - b0));
   const double* Mp = M + (int64_t)pd * FM_BMAX * FM_NM;
-  double S = zeros, SX = 0.0, CN = zeros;
-  for (int k = 0; k < jmax; ++k) {
+  double S = 0.0, SX = 0.0, CN = 0.0;
+  for (int k = lane; k < jmax; k += FM_LANES) {
     const double xb = cen[k] * c;
     if (xb > 800.0) break;                            // later buckets underflow too
     const double t = -hw[k] * c;
@@ -624,10 +652,17 @@ __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restr
     SX += ex * (xb * s0 - t * s1);
     CN += m[0];
   }
+#pragma unroll
+  for (int off = 1; off < FM_LANES; off *= 2) {
+    S += __shfl_xor(S, off, 64);
+    SX += __shfl_xor(SX, off, 64);
+    CN += __shfl_xor(CN, off, 64);
+  }
+  if (lane != 0) return;
   double* o = out + ((int64_t)pd * n_eps + e) * 3;
-  o[0] = S;
+  o[0] = S + zeros;
   o[1] = SX;
-  o[2] = CN;
+  o[2] = CN + zeros;
 }
 
 // ------------------------------------------------------------------ normalisation ------
@@ -1142,6 +1177,13 @@ int memi_knn_select(const void* plan_dev, const memi_plan_info* info, const floa
   return MEMI_OK;
 }
 
+// Parts per tile of the direct sweep (a power of two up to 32): enough blocks to give each CU a few.
+static unsigned sweep_parts(int64_t gx, int64_t tiles) {
+  unsigned parts = 1;
+  while (parts < 32 && gx * tiles * parts < 512) parts *= 2;
+  return parts;
+}
+
 int memi_ferguson_sweep(const void* plan_dev, const memi_plan_info* info, const float* D,
                         const uint32_t* mask, const double* logEps, int n_eps, double* out,
                         void* stream) {
@@ -1161,7 +1203,8 @@ int memi_ferguson_sweep(const void* plan_dev, const memi_plan_info* info, const 
   hipLaunchKernelGGL(k_ferguson_thr, dim3((unsigned)info->n_ftiles), dim3(256), 0, s, v.ftiles,
                      v.pds, D, mask, logEps, n_eps, thr_acc);
   MEMI_CHECK_LAUNCH("k_ferguson_thr");
-  dim3 grid((unsigned)((n_eps + 255) / 256), (unsigned)info->n_ftiles);
+  const unsigned gx = (unsigned)((n_eps + 255) / 256);
+  const dim3 grid(gx, (unsigned)info->n_ftiles, sweep_parts(gx, info->n_ftiles));
   hipLaunchKernelGGL(k_ferguson_sweep, grid, dim3(256), 0, s, v.ftiles, v.pds, D, mask, logEps,
                      n_eps, thr_acc, 2, (const double*)nullptr, out);
   MEMI_CHECK_LAUNCH("k_ferguson_sweep");
@@ -1201,13 +1244,15 @@ int memi_ferguson_moments(const void* plan_dev, const memi_plan_info* info, cons
                      v.ftiles,
                      v.pds, D, mask, gp, M);
   MEMI_CHECK_LAUNCH("k_fer_moments");
-  hipLaunchKernelGGL(k_fer_sweep_moments, dim3((unsigned)((n_eps + 255) / 256), (unsigned)npd),
+  constexpr int EPB = 256 / FM_LANES;        // eps per block
+  hipLaunchKernelGGL(k_fer_sweep_moments, dim3((unsigned)((n_eps + EPB - 1) / EPB), (unsigned)npd),
                      dim3(256), 0, s, logEps, n_eps, gp, M, out);
   MEMI_CHECK_LAUNCH("k_fer_sweep_moments");
   // PDs whose value range or grid step the moments cannot carry (marked by k_fer_grid): the
   // direct sweep, its blocks of every other PD exiting at once
-  hipLaunchKernelGGL(k_ferguson_sweep, dim3((unsigned)((n_eps + 255) / 256),
-                                            (unsigned)info->n_ftiles),
+  const unsigned gx = (unsigned)((n_eps + 255) / 256);
+  hipLaunchKernelGGL(k_ferguson_sweep,
+                     dim3(gx, (unsigned)info->n_ftiles, sweep_parts(gx, info->n_ftiles)),
                      dim3(256), 0, s, v.ftiles, v.pds, D, mask, logEps, n_eps, st, 6,
                      (const double*)gp, out);
   MEMI_CHECK_LAUNCH("k_ferguson_sweep");

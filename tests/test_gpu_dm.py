@@ -399,6 +399,37 @@ def test_ferguson_moments_match_direct_sweep(cuda):
         assert np.max(np.abs(sl1[ok] - sl0[ok])) < 1e-6
 
 
+@pytest.mark.parametrize("n,k,n_eps", [(3, 3, 2), (60, 60, 300), (129, 20, 7), (300, 300, 101),
+                                       (700, 90, 257)])
+def test_ferguson_sweeps_cut_into_parts(cuda, n, k, n_eps):
+    """The direct sweep with its tiles in one to 32 parts and the moment series over eight threads
+    per eps, on small batches and short and long grids, against the float64 sums over the same
+    entries: counts equal, sums within the direct sweep's 1e-7 per term (float32 exp2) and the
+    series' 1e-13."""
+    import torch
+    from manifoldem_python_amd import pipeline as pl
+    plan = _plan(n, k)
+    D = _distance_matrix(n, n).astype(np.float32)
+    Dg = torch.as_tensor(D.ravel(), device=cuda)
+    mask = pl.knn_mask(plan, Dg)
+    bits = mask.cpu().numpy().view(np.uint32).reshape(n, -1)
+    keep = ((bits[:, :, None] >> np.arange(32, dtype=np.uint32)) & 1).reshape(n, -1)[:, :n] > 0
+    keep = keep | keep.T if k < n else np.ones((n, n), bool)
+    v = D.astype(np.float64)[keep]
+    logEps = np.linspace(0.0, 20.0, n_eps)
+    S = {m: pl.ferguson_sums(plan, Dg, mask, logEps, method=m) for m in ("direct", "moments")}
+    mx = np.exp(-v / (2 * np.exp(logEps.max()))).sum()
+    thr = max(-np.log(0.01 * mx / len(v)), 10)
+    for e, le in enumerate(logEps):
+        x = v / (2 * np.exp(le))
+        near = np.abs(x - thr) < 1e-9 * thr
+        ref = np.exp(-x[x < thr]).sum()
+        for m, tol in (("direct", 2e-7), ("moments", 2e-7 if 20.0 / (n_eps - 1) > 0.18 else 1e-12)):
+            if not near.any():
+                assert S[m][2][0, e] == (x < thr).sum(), (m, e)
+            assert abs(S[m][0][0, e] - ref) <= tol * ref, (m, e)
+
+
 @pytest.mark.parametrize("split", [True, False])
 def test_batched_lanczos_many_pds(cuda, split):
     """80 PDs of 40-160 points: the many-PD orthogonalisation (waves walking the live
