@@ -381,6 +381,29 @@ int memi_lanczos_steps_sparse(const void* plan_dev, const memi_plan_info* info,
                               const int32_t* active, double* W, double* H, double* ab,
                               int split, void* stream);
 
+/* nsteps steps from step j0 in one launch, with the outputs of memi_lanczos_steps, for batches
+ * whose workgroups all run at once: each PD is shared by a group of workgroups that exchange its
+ * vectors through memory while they run.
+ * L / ell_* / sparse_pd: as memi_lanczos_steps (ell_col null) or memi_lanczos_steps_sparse.
+ * groups: int32 [n_groups][8] on the device, one entry per workgroup: {PD, first row, end row,
+ * place in the PD's group, workgroups of the group (at most 64), first workgroup of the group, 0,
+ * 0}; the entries of a PD are consecutive and their row ranges cover it.  The caller makes sure
+ * that n_groups is at most the number of CUs the stream may use.  max_rows: the largest row
+ * range.  W: float64 [m * n_rows], kept between the launches of a run (the columns L v_l).
+ * xch: float64 [xch_len >= nsteps (n_rows + n_groups (j0 + nsteps + 3))].  The step's LDS,
+ * 8 (max_n + (j0 + nsteps + 4) max_rows + j0 + nsteps + 1100) bytes, is at most
+ * MEMI_LANCZOS_RUN_LDS, and PDs have at most 4096 rows; j_dev[0] = min(j0 + nsteps, m) afterwards,
+ * as memi_lanczos_steps would leave it.
+ * Every wait between workgroups ends after `spin` polls: then *abort_flag (int32 on the device,
+ * cleared by the launch with j0 = 0) is 1 and the run's V, ab and W are unusable. */
+#define MEMI_LANCZOS_RUN_LDS 155648
+int memi_lanczos_run(const void* plan_dev, const memi_plan_info* info, const void* L, int l_is_f64,
+                     const int32_t* ell_col, const double* ell_val, const int32_t* ell_cnt,
+                     const int32_t* sparse_pd, double* V, double* W, int m, int32_t* j_dev, int j0,
+                     int nsteps, const int32_t* active, double* ab, const int32_t* groups,
+                     int n_groups, int max_rows, double* xch, int64_t xch_len, int32_t* abort_flag,
+                     int spin, void* stream);
+
 /* Convergence check of the batched Lanczos run, the Ritz pairs eigsh(which='LM') returns
  * (sembeddingonFly.py:27-35), entirely on the GPU.  For every active PD with
  * J = min(steps_done, n, m): the k = ks[pd] (<= MEMI_RITZ_KMAX) eigenvalues of largest

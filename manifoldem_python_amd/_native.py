@@ -103,6 +103,9 @@ _SIGS = {
     "memi_kernel_ell": [c_vp, ctypes.POINTER(PlanInfo), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp],
     "memi_lanczos_steps_sparse": [c_vp, ctypes.POINTER(PlanInfo), c_vp, c_vp, c_vp, c_vp, c_vp,
                                   c_vp, c_int, c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_int, c_vp],
+    "memi_lanczos_run": [c_vp, ctypes.POINTER(PlanInfo), c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp,
+                         c_vp, c_int, c_vp, c_int, c_int, c_vp, c_vp, c_vp, c_int, c_int, c_vp,
+                         c_i64, c_vp, c_int, c_vp],
     "memi_tanh_select": [c_vp, c_int, c_int, c_int, c_dbl, c_dbl, c_vp, c_vp, c_vp, c_vp],
     "memi_flow_anisodiff": [c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_int, c_int, c_dbl, c_dbl,
                             c_dbl, c_dbl, c_dbl, c_int, c_vp],
@@ -735,6 +738,54 @@ def lanczos_steps(plan, L, V, m, j_dev, nsteps, active, W, ab, H=None):
          int(L.dtype == torch.float64), _p(V), int(m),
          _p(j_dev), int(nsteps), _p(active), _p(W), None if H is None else _p(H), _p(ab),
          int(H is not None), _stream())
+
+
+LANCZOS_RUN_LDS = 155648         # MEMI_LANCZOS_RUN_LDS
+LANCZOS_RUN_MAX_N = 4096
+LANCZOS_RUN_GMAX = 64            # workgroups per PD
+
+
+def lanczos_run_xch_len(plan, n_groups, j_end, nsteps):
+    """float64 words of memi_lanczos_run's exchange buffer for steps that end at j_end."""
+    return nsteps * (plan.info.n_rows + n_groups * (j_end + 3))
+
+
+def lanczos_run_lds(plan, max_rows, j_end):
+    """Upper bound of memi_lanczos_run's LDS bytes per workgroup for steps that end at j_end."""
+    return 8 * (int(plan.info.max_n) + (j_end + 4) * max_rows + j_end + 1100)
+
+
+def lanczos_run(plan, L, V, Wst, m, j_dev, j0, nsteps, active, ab, groups, max_rows, xch,
+                abort_flag, spin):
+    """nsteps Lanczos steps from step j0 in one launch (memi_lanczos_run).  L as in
+    ``lanczos_steps``; groups: int32 (n_groups, 8) device table, one row per workgroup; abort_flag:
+    int32 device tensor, nonzero afterwards when a bounded wait ran out (the run is then
+    unusable)."""
+    I = plan.info
+    _need(V.numel() >= m * I.n_rows and Wst.numel() >= m * I.n_rows and
+          V.dtype == Wst.dtype == torch.float64 and ab.numel() >= I.n_pd * m * 2 and
+          active.dtype == torch.int32 and active.numel() >= I.n_pd, "lanczos_run: buffers")
+    _need(groups.dtype == torch.int32 and groups.dim() == 2 and groups.shape[1] == 8,
+          "lanczos_run: groups must be int32 (n_groups, 8)")
+    _need(xch.dtype == torch.float64 and j_dev.dtype == torch.int32 and j_dev.numel() >= 2 and
+          abort_flag.dtype == torch.int32, "lanczos_run: xch float64, j_dev and abort_flag int32")
+    col = val = cnt = sel = Ld = None
+    if isinstance(L, tuple):
+        col, val, cnt = L[:3]
+        if len(L) == 5:
+            sel, Ld = L[3], L[4]
+    else:
+        Ld = L
+    _need(Ld is None or (Ld.numel() >= I.d_elems and
+                         Ld.dtype in (torch.float32, torch.float64)), "lanczos_run: L")
+    _need(sel is None or (sel.dtype == torch.int32 and sel.numel() >= I.n_pd and
+                          Ld.dtype == torch.float64), "lanczos_run: sel")
+    opt = lambda t: None if t is None else _p(t)
+    call("memi_lanczos_run", _p(plan.dev), ctypes.byref(plan.info), opt(Ld),
+         int(Ld is None or Ld.dtype == torch.float64), opt(col), opt(val), opt(cnt), opt(sel),
+         _p(V), _p(Wst), int(m), _p(j_dev), int(j0), int(nsteps), _p(active), _p(ab), _p(groups),
+         int(groups.shape[0]), int(max_rows), _p(xch), int(xch.numel()), _p(abort_flag), int(spin),
+         _stream())
 
 
 RITZ_KMAX = 16

@@ -536,6 +536,355 @@ __global__ void k_step_advance(int32_t* __restrict__ jp) {
   if (threadIdx.x == 0) jp[0] = jp[0] + 1;
 }
 
+// ---- a block of steps in one launch --------------------------------------------------------
+// For batches whose workgroups are all resident at once (at most one per CU): every PD has a
+// group of G workgroups, each owning the rows [r0, r1) of its kernel and basis, and the group
+// walks through `nsteps` steps on its own.  Per step, with u the vector the last step published
+// (v_j itself in a launch's first step, afterwards w' of the step before, not yet divided by beta
+// nor stripped of V h):
+//   y = L u on the own rows, turned into L v_j by linearity, (y - sum_l h_l (L v_l)) / beta, from
+//     the stored columns L v_l (Wst);
+//   alpha = v_j . y over the group (first exchange);
+//   w' = (y - alpha v_j) - beta_{j-1} v_{j-1}, published (second exchange), and with it the own
+//     rows' parts of h = V^T w' and w'.w';
+//   beta^2 = w'.w' - ||h||^2, v_{j+1} = (w' - V h) / beta on the own rows.
+// The arithmetic is that of the three-launch step but for the order of the sums.
+//
+// Exchange.  Values travel through memory as single float64 words, written and read by relaxed
+// agent-scope atomics (which bypass the XCDs' non-coherent caches) into slots that hold an
+// all-ones pattern until written, one set of slots per step: the arrival of a value is its own
+// flag, so a round trip replaces a store, a counter and a read, and no fence writes back or
+// invalidates a cache (a grid barrier with agent-scope fences cost ~40 us here).  A value that
+// is itself the all-ones pattern (a NaN no operation produces) is published as the usual NaN.
+// Every wait is bounded by `spin` polls; a workgroup that runs out raises *abort_flag, which the
+// others poll too, and the launch ends with the run unusable: the caller starts over with the
+// launches above.
+//
+// Bound: latency -- the two exchanges (~2.5 us each), the rows of L from the XCDs' L2s (one round
+// of loads per step) and the barriers of an eight-wave workgroup.  Per step, against the three
+// launches above with their gaps: one PD of 200 rows 7.2 us against 14, of 1273 dense rows 9.7
+// against 20, of 2000 rows of ~300 nonzeros 10.5 against 21; 64 PDs of 100 to 1700 rows, four
+// workgroups each on average, 29 against 62.
+constexpr int LR_NT = 512;                  // threads per workgroup
+constexpr int LR_WAVES = LR_NT / 64;
+constexpr int LR_GMAX = 64;                 // workgroups per group
+constexpr int LR_PARTS = LR_NT / 128;       // threads that share a column's sum over the group
+constexpr int LR_UMAX = 8;                  // elements of u per thread: n <= 4096
+constexpr unsigned long long LR_EMPTY = ~0ull;
+
+struct LrGroup {
+  int32_t pd, r0, r1, gi, G, wg0;           // this workgroup's rows; its place in the group; the
+  int32_t pad0, pad1;                       // group's first workgroup
+};
+
+__device__ __forceinline__ unsigned long long lr_load(const double* p) {
+  return __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void lr_publish(double* p, double v) {
+  unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  if (b == LR_EMPTY) b = 0x7FF8000000000000ull;
+  __hip_atomic_store((unsigned long long*)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits for the values at the N addresses (null: none), all loads in flight together; false when
+// the bound or the abort flag ends the wait.
+template <int N>
+__device__ __forceinline__ bool lr_wait(const double* const (&p)[N], double (&v)[N], int spin,
+                                        const int32_t* abort_flag) {
+  for (int it = 0;; ++it) {
+    unsigned long long b[N];
+    bool all = true;
+#pragma unroll
+    for (int e = 0; e < N; ++e) b[e] = p[e] ? lr_load(p[e]) : 0ull;
+#pragma unroll
+    for (int e = 0; e < N; ++e) all = all && b[e] != LR_EMPTY;
+    if (all) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] = __longlong_as_double((long long)b[e]);
+      return true;
+    }
+    if (it >= spin) return false;
+    if ((it & 63) == 63 &&
+        __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return false;
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+// Empties the exchange slots of the next launch and sets the step index it will reach.
+__global__ void k_lanczos_run_begin(unsigned long long* __restrict__ xch, int64_t len,
+                                    int32_t* __restrict__ jp, int j_end,
+                                    int32_t* __restrict__ abort_flag, int clear_abort) {
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int64_t t = t0; t < len; t += (int64_t)gridDim.x * blockDim.x) xch[t] = LR_EMPTY;
+  if (t0 == 0) {
+    jp[0] = j_end;
+    if (clear_abort) *abort_flag = 0;
+  }
+}
+
+// y[r LR_WAVES] = row r of L (R rows, dr elements apart from d0) times u: dense rows, or the first
+// cnt[r LR_WAVES] nonzeros of sparse ones; 16 loads in flight per lane.
+template <int R, typename T>
+__device__ __forceinline__ void lr_rows(bool sparse, const T* __restrict__ L,
+                                        const int32_t* __restrict__ col,
+                                        const double* __restrict__ val,
+                                        const int32_t* __restrict__ cnt, int64_t d0, int64_t dr,
+                                        const double* u, int n, int lane, double* y) {
+  constexpr int Q = R == 1 ? 8 : R == 2 ? 8 : 4;       // 64-wide pieces of a row per round
+  double s[R] = {};
+  if (sparse) {
+    constexpr int QS = R == 1 ? 4 : 2;
+    int c[R], cm = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      c[r] = cnt[r * LR_WAVES];
+      cm = max(cm, c[r]);
+    }
+    for (int q = lane; q < cm; q += 64 * QS) {
+      int ci[R][QS];
+      double va[R][QS];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < QS; ++e) {
+          const bool in = q + 64 * e < c[r];
+          const int64_t o = d0 + r * dr + (in ? q + 64 * e : 0);
+          ci[r][e] = in ? col[o] : 0;
+          va[r][e] = in ? val[o] : 0.0;
+        }
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < QS; ++e)
+          if (q + 64 * e < c[r]) s[r] += va[r][e] * u[ci[r][e]];
+    }
+  } else {
+    const T* p = L + d0;
+    int c = lane;
+    for (; c + 64 * (Q - 1) < n; c += 64 * Q) {
+      T a[R][Q];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < Q; ++e) a[r][e] = p[r * dr + c + 64 * e];
+#pragma unroll
+      for (int e = 0; e < Q; ++e) {
+        const double x = u[c + 64 * e];
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r] += (double)a[r][e] * x;
+      }
+    }
+    if (c < n) {                             // the last, partial round, its loads together too
+      T a[R][Q];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < Q; ++e) a[r][e] = p[r * dr + min(c + 64 * e, n - 1)];
+#pragma unroll
+      for (int e = 0; e < Q; ++e)
+        if (c + 64 * e < n) {
+          const double x = u[c + 64 * e];
+#pragma unroll
+          for (int r = 0; r < R; ++r) s[r] += (double)a[r][e] * x;
+        }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const double v = wave_total(s[r]);
+    if (lane == 0) y[r * LR_WAVES] = v;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(LR_NT) void k_lanczos_run(
+    const LrGroup* __restrict__ groups, const memi_pd_desc* __restrict__ pds,
+    const T* __restrict__ L, const int32_t* __restrict__ ell_col,
+    const double* __restrict__ ell_val, const int32_t* __restrict__ ell_cnt,
+    const int32_t* __restrict__ sel, double* V, double* Wst, int m, int j0, int nsteps, int n_wg,
+    int64_t n_rows, const int32_t* __restrict__ active, double* ab, double* xch, int hs,
+    int w_in_lds, int spin, int32_t* abort_flag) {
+  extern __shared__ double lds[];
+  const LrGroup g = groups[blockIdx.x];
+  if (!active[g.pd]) return;
+  const memi_pd_desc P = pds[g.pd];
+  const int n = P.n, nr = g.r1 - g.r0;
+  const int j_end = min(j0 + nsteps, min(n, m));
+  if (j0 >= j_end) return;                  // the whole space already
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool sparse = ell_col && !(sel && !sel[g.pd]);
+  double* u = lds;                          // [n]
+  double* yl = u + n;                       // [nr] y, then w'
+  double* cw = yl + nr;                     // [nr] sum_l h_l (L v_l)
+  double* h = cw + nr;                      // [hs]
+  double* red = h + hs;                     // [LR_PARTS][128]
+  double* sc = red + LR_PARTS * 128;        // alpha; sc[1] as int: a wait failed
+  int* bad = (int*)(sc + 1);
+  double* Vl = sc + 2;                      // [columns][nr]: the own rows of the basis
+  double* Wl = Vl + (j0 + nsteps + 1) * nr; // and of the columns L v_l, when w_in_lds
+  double* xw = xch + P.row0;                                           // [nsteps][n_rows]
+  double* xa = xch + (int64_t)nsteps * n_rows;                         // [nsteps][n_wg]
+  double* xh = xa + (int64_t)nsteps * n_wg;                            // [nsteps][n_wg][hs]
+  double* Vg = V + (int64_t)m * P.row0;
+  double* Wg = Wst + (int64_t)m * P.row0;
+  for (int e = tid; e < (j0 + 1) * nr; e += LR_NT) {
+    const int l = e / nr, i = e - l * nr;
+    Vl[e] = Vg[(int64_t)l * n + g.r0 + i];
+    if (w_in_lds && l < j0) Wl[e] = Wg[(int64_t)l * n + g.r0 + i];
+  }
+  for (int k = tid; k < n; k += LR_NT) u[k] = Vg[(int64_t)j0 * n + k];
+  // a launch queued behind one that gave up does nothing
+  if (tid == 0) *bad = __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double bprev = j0 > 0 ? ab[((int64_t)g.pd * m + j0 - 1) * 2 + 1] : 0.0;
+  double inv = 1.0;                         // 1 / beta of the step before
+  __syncthreads();
+  for (int j = j0; j < j_end && !*bad; ++j) {
+    const int t = j - j0;
+    // y = L u: up to four rows per wave at a time, u from LDS
+    for (int ib = w; ib < nr; ib += 4 * LR_WAVES) {
+      const int left = (nr - ib + LR_WAVES - 1) / LR_WAVES;
+      const int64_t d0 = P.d_off + (int64_t)(g.r0 + ib) * n, dr = (int64_t)LR_WAVES * n;
+      const int32_t* cnt = ell_cnt + P.row0 + g.r0 + ib;
+      double* y = yl + ib;
+      if (left >= 4) lr_rows<4>(sparse, L, ell_col, ell_val, cnt, d0, dr, u, n, lane, y);
+      else if (left == 3) lr_rows<3>(sparse, L, ell_col, ell_val, cnt, d0, dr, u, n, lane, y);
+      else if (left == 2) lr_rows<2>(sparse, L, ell_col, ell_val, cnt, d0, dr, u, n, lane, y);
+      else lr_rows<1>(sparse, L, ell_col, ell_val, cnt, d0, dr, u, n, lane, y);
+    }
+    __syncthreads();
+    const double* vj = Vl + (int64_t)j * nr;
+    // L v_j on the own rows and the group's alpha, by the first wave
+    if (w == 0) {
+      double a = 0.0;
+      for (int i = lane; i < nr; i += 64) {
+        double y = yl[i];
+        if (t > 0) {
+          y = (y - cw[i]) * inv;
+          yl[i] = y;
+        }
+        Wg[(int64_t)j * n + g.r0 + i] = y;
+        if (w_in_lds) Wl[j * nr + i] = y;
+        a += vj[i] * y;
+      }
+      a = wave_total(a);
+      if (lane == 0) lr_publish(xa + (int64_t)t * n_wg + g.wg0 + g.gi, a);
+      const double* const p[1] = {lane < g.G ? xa + (int64_t)t * n_wg + g.wg0 + lane : nullptr};
+      double v[1];
+      const bool ok = lr_wait<1>(p, v, spin, abort_flag);
+      if (!ok) *bad = 1;
+      a = wave_total(ok && lane < g.G ? v[0] : 0.0);
+      if (lane == 0) sc[0] = a;
+    }
+    __syncthreads();
+    if (*bad) break;
+    const double alpha = sc[0];
+    const double* vjm = j > 0 ? vj - nr : vj;
+    for (int i = tid; i < nr; i += LR_NT) {
+      const double x = (yl[i] - alpha * vj[i]) - (j > 0 ? bprev * vjm[i] : 0.0);
+      yl[i] = x;
+      lr_publish(xw + (int64_t)t * n_rows + g.r0 + i, x);
+    }
+    __syncthreads();
+    // the own rows' parts of h (columns 0..j) and of w'.w' (column j + 1): eight lanes each
+    double* xo = xh + ((int64_t)t * n_wg + g.wg0 + g.gi) * hs;
+    for (int cb = 0; cb < j + 2; cb += LR_NT / 8) {
+      const int c = cb + (tid >> 3);
+      double s = 0.0;
+      if (c < j + 2) {
+        const double* vc = c <= j ? Vl + (int64_t)c * nr : yl;
+        for (int i = tid & 7; i < nr; i += 8) s += vc[i] * yl[i];
+      }
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s += __shfl_xor(s, 4, 64);
+      if (c < j + 2 && (tid & 7) == 0) lr_publish(xo + c, s);
+    }
+    // the group's h and w', the loads of both in flight together: thread (c, part) takes every
+    // LR_PARTS-th workgroup's word of column c
+    for (int cb = 0; cb < j + 2; cb += 128) {
+      const int c = cb + (tid & 127), part = tid >> 7;
+      const double* p[LR_GMAX / LR_PARTS + LR_UMAX];
+      double v[LR_GMAX / LR_PARTS + LR_UMAX];
+#pragma unroll
+      for (int e = 0; e < LR_GMAX / LR_PARTS; ++e) {
+        const int q = part + e * LR_PARTS;
+        p[e] = c < j + 2 && q < g.G ? xh + ((int64_t)t * n_wg + g.wg0 + q) * hs + c : nullptr;
+      }
+#pragma unroll
+      for (int e = 0; e < LR_UMAX; ++e) {
+        const int k = tid + e * LR_NT;
+        p[LR_GMAX / LR_PARTS + e] = cb == 0 && k < n ? xw + (int64_t)t * n_rows + k : nullptr;
+      }
+      if (!lr_wait(p, v, spin, abort_flag)) *bad = 1;
+      double s = 0.0;
+#pragma unroll
+      for (int e = 0; e < LR_GMAX / LR_PARTS; ++e)
+        if (p[e]) s += v[e];
+      red[part * 128 + (tid & 127)] = s;
+#pragma unroll
+      for (int e = 0; e < LR_UMAX; ++e)
+        if (p[LR_GMAX / LR_PARTS + e]) u[tid + e * LR_NT] = v[LR_GMAX / LR_PARTS + e];
+      __syncthreads();
+      if (tid < 128 && c < j + 2) {
+        double x = 0.0;
+#pragma unroll
+        for (int q = 0; q < LR_PARTS; ++q) x += red[q * 128 + tid];
+        h[c] = x;
+      }
+      __syncthreads();
+    }
+    if (*bad) break;
+    double hh = 0.0;                        // every wave sums ||h||^2 in the same order
+    for (int l = lane; l <= j; l += 64) hh += h[l] * h[l];
+    hh = wave_total(hh);
+    const double beta = sqrt(fmax(h[j + 1] - hh, 0.0));
+    inv = beta > 0.0 ? 1.0 / beta : 0.0;
+    // v_{j+1} and the next step's sum_l h_l (L v_l) on the own rows: sixteen lanes per row
+    for (int ib = 0; ib < nr; ib += LR_NT / 16) {
+      const int i = ib + (tid >> 4), sub = tid & 15;
+      double sv = 0.0, sw = 0.0;
+      if (i < nr) {
+        if (w_in_lds) {
+#pragma unroll 4
+          for (int l = sub; l <= j; l += 16) {
+            sv += Vl[l * nr + i] * h[l];
+            sw += Wl[l * nr + i] * h[l];
+          }
+        } else {
+#pragma unroll 4
+          for (int l = sub; l <= j; l += 16) {
+            sv += Vl[l * nr + i] * h[l];
+            sw += Wg[(int64_t)l * n + g.r0 + i] * h[l];
+          }
+        }
+      }
+#pragma unroll
+      for (int off = 1; off < 16; off *= 2) {
+        sv += __shfl_xor(sv, off, 64);
+        sw += __shfl_xor(sw, off, 64);
+      }
+      if (i < nr && sub == 0) {
+        const double x = (yl[i] - sv) * inv;
+        cw[i] = sw;
+        Vl[(j + 1) * nr + i] = x;
+        if (j + 1 < m) Vg[(int64_t)(j + 1) * n + g.r0 + i] = x;
+      }
+    }
+    if (g.gi == 0 && tid == 0) {
+      ab[((int64_t)g.pd * m + j) * 2 + 0] = alpha + h[j];
+      ab[((int64_t)g.pd * m + j) * 2 + 1] = beta;
+    }
+    bprev = beta;
+    __syncthreads();
+  }
+  if (*bad && tid == 0)
+    __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---- convergence check: Ritz pairs of the tridiagonal T_p on the GPU -----------------------
 // One workgroup per active PD with J = min(steps, n, m) Lanczos steps.
 //  1. candidates: the k smallest and k largest eigenvalues of T (all J when J <= 2k), each by
@@ -1053,6 +1402,55 @@ int memi_lanczos_steps_sparse(const void* plan_dev, const memi_plan_info* info,
                  "memi_lanczos_steps_sparse: null pointer (a selection needs the dense L)");
   return lanczos_steps_impl(plan_dev, info, L, 1, ell_col, ell_val, ell_cnt, sparse_pd, V, m,
                             j_dev, nsteps, active, W, H, ab, split, stream);
+}
+
+int memi_lanczos_run(const void* plan_dev, const memi_plan_info* info, const void* L, int l_is_f64,
+                     const int32_t* ell_col, const double* ell_val, const int32_t* ell_cnt,
+                     const int32_t* sparse_pd, double* V, double* W, int m, int32_t* j_dev, int j0,
+                     int nsteps, const int32_t* active, double* ab, const int32_t* groups,
+                     int n_groups, int max_rows, double* xch, int64_t xch_len, int32_t* abort_flag,
+                     int spin, void* stream) {
+  MEMI_CHECK_ARG(plan_dev && info && (L || ell_col) && V && W && j_dev && active && ab && groups &&
+                     xch && abort_flag,
+                 "memi_lanczos_run: null pointer");
+  MEMI_CHECK_ARG(!ell_col || (ell_val && ell_cnt && l_is_f64 && (!sparse_pd || L)),
+                 "memi_lanczos_run: a sparse kernel needs its values and counts, a selection the "
+                 "dense float64 L");
+  MEMI_CHECK_ARG(ell_col || !sparse_pd, "memi_lanczos_run: a selection without sparse rows");
+  MEMI_CHECK_ARG(m >= 2 && m <= 4096 && j0 >= 0 && nsteps >= 1 && j0 + nsteps <= m + nsteps &&
+                     n_groups >= 1 && max_rows >= 1 && spin >= 0,
+                 "memi_lanczos_run: bad m=%d j0=%d nsteps=%d n_groups=%d", m, j0, nsteps, n_groups);
+  MEMI_CHECK_ARG(info->max_n <= LR_UMAX * LR_NT, "memi_lanczos_run: PDs of at most %d rows (%d)",
+                 LR_UMAX * LR_NT, info->max_n);
+  const int hs = j0 + nsteps + 2;
+  const int64_t len = (int64_t)nsteps * (info->n_rows + (int64_t)n_groups * (1 + hs));
+  MEMI_CHECK_ARG(xch_len >= len, "memi_lanczos_run: exchange buffer %lld < %lld",
+                 (long long)xch_len, (long long)len);
+  int64_t lds = 8 * ((int64_t)info->max_n + 2 * max_rows + hs + LR_PARTS * 128 + 2 +
+                           (int64_t)(j0 + nsteps + 1) * max_rows);
+  MEMI_CHECK_ARG(lds <= MEMI_LANCZOS_RUN_LDS, "memi_lanczos_run: %lld bytes of LDS for step %d",
+                 (long long)lds, j0 + nsteps);
+  if (info->n_pd == 0) return MEMI_OK;
+  // the columns L v_l stay in LDS too where there is room (else they are read from the L2)
+  const int64_t more = 8 * (int64_t)(j0 + nsteps) * max_rows;
+  const int w_in_lds = lds + more <= MEMI_LANCZOS_RUN_LDS;
+  if (w_in_lds) lds += more;
+  hipStream_t s = (hipStream_t)stream;
+  const memi_pd_desc* pds = (const memi_pd_desc*)((const char*)plan_dev + info->off_pds);
+  hipLaunchKernelGGL(k_lanczos_run_begin, dim3(grid_for(len, 256, 1024)), dim3(256), 0, s,
+                     (unsigned long long*)xch, len, j_dev, std::min(j0 + nsteps, m), abort_flag,
+                     (int)(j0 == 0));
+  MEMI_CHECK_LAUNCH("k_lanczos_run_begin");
+#define MEMI_LANCZOS_RUN(T)                                                                    \
+  hipLaunchKernelGGL(k_lanczos_run<T>, dim3((unsigned)n_groups), dim3(LR_NT), (size_t)lds, s,  \
+                     (const LrGroup*)groups, pds, (const T*)L, ell_col, ell_val, ell_cnt,      \
+                     sparse_pd, V, W, m, j0, nsteps, n_groups, info->n_rows, active, ab, xch,  \
+                     hs, w_in_lds, spin, abort_flag)
+  if (l_is_f64) MEMI_LANCZOS_RUN(double);
+  else MEMI_LANCZOS_RUN(float);
+#undef MEMI_LANCZOS_RUN
+  MEMI_CHECK_LAUNCH("k_lanczos_run");
+  return MEMI_OK;
 }
 
 int memi_kernel_ell(const void* plan_dev, const memi_plan_info* info, const double* L,

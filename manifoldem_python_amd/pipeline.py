@@ -574,6 +574,68 @@ def _next_check_gap(j, res, thmax, active, tol, step, hist, slack=0.6, cap=4):
     return gap, (j, lr), last
 
 
+# memi_lanczos_run: entries of the kernel per workgroup (embeddings of 200, 1273 and 2000 rows and
+# of eight PDs took 1.63, 1.87, 1.95 and 1.75 ms with 4096, 1.75, 1.89, 1.95 and 1.95 with 16384,
+# 1.90, 2.19, 2.63 and 2.57 with 65536), the basis columns its LDS always holds, and the polls
+# after which a wait between workgroups gives up (each takes about a microsecond).
+RUN_WORK = 4096
+RUN_COLUMNS = 96
+RUN_SPIN = 1 << 18
+
+
+def run_groups(ns, work, max_n, cus):
+    """Workgroups of memi_lanczos_run: an int32 (n_groups, 8) table giving every PD of sizes ns a
+    group of workgroups by its kernel entries (work), at most `cus` in all (they must all be
+    resident, one per CU); None when the batch does not fit.  A workgroup's rows are few enough
+    for RUN_COLUMNS of its basis in LDS."""
+    ns, work = np.asarray(ns, dtype=np.int64), np.asarray(work, dtype=np.float64)
+    rows = (nat.LANCZOS_RUN_LDS // 8 - int(max_n) - 1200 - RUN_COLUMNS) // (RUN_COLUMNS + 4)
+    if max_n > nat.LANCZOS_RUN_MAX_N or rows < 1 or len(ns) > cus:
+        return None
+    least = -(-ns // rows)
+    if least.max() > nat.LANCZOS_RUN_GMAX or least.sum() > cus:
+        return None
+    want = np.clip(np.ceil(work / RUN_WORK).astype(np.int64), 1, nat.LANCZOS_RUN_GMAX)
+    G = np.maximum(least, np.minimum(want, ns))
+    if G.sum() > cus:                    # shares of the CUs by work, the remainder to the largest
+        G = np.maximum(least, np.minimum(G, np.floor(cus * work / work.sum()).astype(np.int64)))
+        while G.sum() > cus:
+            G[np.argmin(np.where(G > least, work / G, np.inf))] -= 1
+    out = np.zeros((int(G.sum()), 8), dtype=np.int32)
+    wg = 0
+    for p, (n, q) in enumerate(zip(ns, G)):
+        edge = np.arange(q + 1) * n // q
+        r = out[wg:wg + q]
+        r[:, 0], r[:, 1], r[:, 2] = p, edge[:-1], edge[1:]
+        r[:, 3], r[:, 4], r[:, 5] = np.arange(q), q, wg
+        wg += int(q)
+    return out
+
+
+def _run_state(plan, L, m, dev):
+    """Buffers of memi_lanczos_run for the plan, or None when its workgroups do not all fit on the
+    CUs (``plan.cu_limit`` of them, when a caller keeps the plan's work on a part of the GPU)."""
+    ns = plan.ns.astype(np.int64)
+    per_row = ns.astype(np.float64)
+    if isinstance(L, tuple):
+        few = plan.ks * SPARSE_RATIO <= ns if len(L) == 5 else np.ones(len(ns), dtype=bool)
+        per_row = np.where(few, 3.0 * plan.ks, per_row)   # ~2 k nonzeros of 12 bytes
+    cus = getattr(plan, "cu_limit", None) or \
+        torch.cuda.get_device_properties(dev).multi_processor_count
+    table = run_groups(ns, ns * per_row, int(plan.info.max_n), int(cus))
+    if table is None:
+        return None
+    n_groups, max_rows = len(table), int((table[:, 2] - table[:, 1]).max())
+    # steps per launch: as many as keep the exchange buffer (emptied before every launch) small
+    most = int(max(8, min(40, 500_000 // (plan.info.n_rows + 64 * n_groups) // 8 * 8)))
+    last = (nat.LANCZOS_RUN_LDS // 8 - int(plan.info.max_n) - 1100 - 4 * max_rows) // (max_rows + 1)
+    last = min(last, m + most)
+    return dict(groups=torch.as_tensor(table, device=dev), max_rows=max_rows, most=most, last=last,
+                W=torch.empty(m * plan.info.n_rows, dtype=torch.float64, device=dev),
+                xch=torch.empty(nat.lanczos_run_xch_len(plan, n_groups, last, most),
+                                dtype=torch.float64, device=dev))
+
+
 def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20261202,
                  split=None, check="gpu", graph=True, full=False):
     """Largest-magnitude eigenpairs of every PD's kernel block of L (float64 or float32) with
@@ -590,7 +652,9 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     not predicted to end the run) or "host" (scipy tridiagonal eigensolver per PD, every 32
     steps by default).  graph: the launches of one block of
     check_every steps are captured once in a HIP graph and replayed (the step index lives on
-    the device).  Returns a list of (lam, V (n x k) numpy, steps, max residual); with full,
+    the device).  With split left open and check "gpu", batches whose workgroups all fit on the
+    GPU at once run each block of steps in one launch instead (memi_lanczos_run), and fall back to
+    the launches above if a wait between its workgroups ever runs out.  Returns a list of (lam, V (n x k) numpy, steps, max residual); with full,
     also the (n_rows x kmax) array the V are row blocks of."""
     sparse = isinstance(L, tuple)               # (col, val, cnt) of nat.kernel_ell
     dev = (L[1] if sparse else L).device
@@ -601,6 +665,7 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     if m is None:
         m = int(min(ns.max(), 512))
     m = int(max(2, min(m, ns.max())))
+    may_run = split is None and check == "gpu"
     if split is None:
         split = npd < 128 or int(ns.max()) > 1024
     if check_every is None:
@@ -615,7 +680,7 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     # buffers (and the captured block of steps) persist on the plan between calls with the
     # same L buffer and settings, so repeated embeddings only replay the graph
     key = (tuple(t.data_ptr() for t in L) if sparse else (L.data_ptr(), L.numel(), str(L.dtype)),
-           m, bool(split), check_every, bool(graph), check)
+           m, bool(split), check_every, bool(graph), check, may_run)
     st = getattr(plan, "_lanczos", None)
     if st is None or st["key"] != key:
         st = dict(key=key)
@@ -631,17 +696,20 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
             st["steps"] = torch.zeros(npd, dtype=torch.int32, device=dev)
             st["res"] = torch.zeros(npd, dtype=torch.float64, device=dev)
             st["piv"] = torch.empty(npd * K * 2 * m, dtype=torch.float64, device=dev)
-            st["summary"] = torch.zeros(3 * npd, dtype=torch.float64, device=dev)
-            st["summary_h"] = torch.zeros(3 * npd, dtype=torch.float64, pin_memory=True)
+            # the word after the summary is memi_lanczos_run's abort flag: one copy brings both
+            st["summary"] = torch.zeros(3 * npd + 1, dtype=torch.float64, device=dev)
+            st["summary_h"] = torch.zeros(3 * npd + 1, dtype=torch.float64, pin_memory=True)
             st["summary_ev"] = torch.cuda.Event()
         st["graph"] = None
-        if graph:
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                nat.lanczos_steps(plan, L, st["V"], m, st["j"], check_every, st["active"],
-                                  st["W"], st["ab"], H=st["H"])
-            st["graph"] = g
+        st["run"] = _run_state(plan, L, m, dev) if may_run else None
         plan._lanczos = st
+    run = st["run"]
+    if graph and run is None and st["graph"] is None:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            nat.lanczos_steps(plan, L, st["V"], m, st["j"], check_every, st["active"],
+                              st["W"], st["ab"], H=st["H"])
+        st["graph"] = g
     V, W, H, ab, active, j_dev, g = (st["V"], st["W"], st["H"], st["ab"], st["active"], st["j"],
                                      st["graph"])
     if check == "gpu":
@@ -672,11 +740,28 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     ks_t = st["ks_t"]
     steps = np.minimum(ns, m)
     out = [None] * npd
-    def block():
-        if g is not None:
+    if run is not None:
+        abort_flag = st["summary"][3 * npd:].view(torch.int32)
+
+    def block(j, target):
+        """Queues steps from j: a block of check_every, or the blocks up to target in one launch.
+        Returns the new step count."""
+        if run is not None:
+            q = max(1, min(-(-(target - j) // check_every), run["most"] // check_every))
+            if j + q * check_every > run["last"]:
+                q = 1
+            nsteps = q * check_every
+            if nsteps <= run["most"] and j + nsteps <= run["last"]:
+                nat.lanczos_run(plan, L, V, run["W"], m, j_dev, j, nsteps, active, ab,
+                                run["groups"], run["max_rows"], run["xch"], abort_flag, RUN_SPIN)
+                return min(m, j + nsteps)
+            # the basis has outgrown the workgroups' LDS: the rest of the run step by step
+            nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
+        elif g is not None:
             g.replay()
         else:
             nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
+        return min(m, j + check_every)
 
     j = 0                            # steps queued on the stream
     jc = 0                           # step count of the last check
@@ -686,8 +771,7 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     while active_h.any():
         target = first_check if jc == 0 else min(m, jc + gap)
         while j < target:
-            block()
-            j = min(m, j + check_every)
+            j = block(j, target)
         jc = j
         if check == "gpu":
             # the check writes {active, largest residual, max |theta|} per PD; one async copy
@@ -700,10 +784,15 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
             st["summary_h"].copy_(st["summary"], non_blocking=True)
             st["summary_ev"].record()
             if jc < m and (last is None or last > jc):
-                block()
-                j = min(m, j + check_every)
+                j = block(j, j + check_every)
             st["summary_ev"].synchronize()
-            h = st["summary_h"].numpy().reshape(3, npd)
+            if run is not None and st["summary_h"][3 * npd:].view(torch.int32)[0]:
+                # a wait between workgroups ran out (work on other streams held their CUs): this
+                # plan goes back to one launch per phase of a step, from the start
+                st["run"] = None
+                return lanczos_eigs(plan, L, ks, m, tol, check_every, seed, None, check, graph,
+                                    full)
+            h = st["summary_h"].numpy()[:3 * npd].reshape(3, npd)
             active_h = h[0].astype(np.int32)
             gap, hist, last = _next_check_gap(jc, h[1], h[2], active_h, tol, check_every, hist)
             continue

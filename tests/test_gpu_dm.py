@@ -460,3 +460,93 @@ def test_batched_lanczos_many_pds(cuda, split):
         np.testing.assert_allclose(lam, w[sel], atol=1e-9)
         for c in range(9):
             assert abs(abs(np.dot(Y[:, c], U[:, sel[c]])) - 1) < 1e-6, (p, c)
+
+
+def _kernel(cuda, ns, ks, dtype="float64"):
+    """(plan, L) of a batch: the normalised kernels of curved point sets, kNN-cut to ks."""
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    D = [_distance_matrix(n, 60 + i) for i, n in enumerate(ns)]
+    rows0 = np.concatenate(([0], np.cumsum(ns)[:-1]))
+    plan = nat.Plan(rows0, ns, ks, chunks=1)
+    flat = torch.as_tensor(np.concatenate([d.astype(np.float32).ravel() for d in D]),
+                           device=cuda)
+    mask = pl.knn_mask(plan, flat)
+    sigma = torch.as_tensor([np.sqrt(np.median(d)) for d in D], device=cuda)
+    L = torch.empty(plan.info.d_elems, dtype=getattr(torch, dtype), device=cuda)
+    deg = torch.empty(2 * plan.info.n_rows, dtype=torch.float64, device=cuda)
+    nat.markov_normalize(plan, flat, mask, sigma, L, deg)
+    return plan, L
+
+
+def _check_eigs(plan, L, res, kk):
+    for p in range(plan.npd):
+        A = plan.block(L, p).double().cpu().numpy()
+        w, U = np.linalg.eigh(A)
+        sel = np.argsort(-np.abs(w), kind="stable")[:kk[p]]
+        sel = sel[np.argsort(-w[sel], kind="stable")]
+        lam, Y, J, r = res[p]
+        np.testing.assert_allclose(lam, w[sel], atol=1e-9)
+        for c in range(kk[p]):
+            assert abs(abs(np.dot(Y[:, c], U[:, sel[c]])) - 1) < 1e-6, (p, c)
+
+
+@pytest.mark.parametrize("ns,ks,kk,dtype", [
+    ([4], [4], [2], "float64"), ([65], [65], [9], "float32"), ([200], [200], [9], "float64"),
+    ([20, 333, 16], [20, 120, 16], [8, 14, 6], "float64"), ([1273], [1273], [16], "float64"),
+    ([700, 130, 64, 1], [70, 130, 20, 1], [11, 9, 9, 1], "float64"),
+    (list(range(40, 160, 3)), list(range(40, 160, 3)), [9] * 40, "float64")])
+def test_lanczos_run_matches_dense(cuda, ns, ks, kk, dtype):
+    """The launches that hold a block of steps (one to 64 workgroups per PD exchanging vectors
+    through memory; dense, sparse and mixed kernels; PDs that exhaust their space) against dense
+    eigh, and the step counts and eigenvalues of the launch-per-phase steps."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    import torch
+    plan, L = _kernel(cuda, ns, ks, dtype)
+    few = [4 * k <= n for n, k in zip(ns, ks)]
+    Lx = L
+    if any(few):
+        ell = (torch.empty(plan.info.d_elems, dtype=torch.int32, device=cuda),
+               torch.empty(plan.info.d_elems, dtype=torch.float64, device=cuda),
+               torch.empty(plan.info.n_rows, dtype=torch.int32, device=cuda))
+        sel = torch.as_tensor(np.asarray(few, dtype=np.int32), device=cuda)
+        nat.kernel_ell(plan, L, *ell, sel=sel)
+        Lx = ell + (sel, L)
+    for again in range(2):                     # a second run on the kept buffers
+        res = pl.lanczos_eigs(plan, Lx, kk)
+        assert plan._lanczos["run"] is not None
+        _check_eigs(plan, L, res, kk)
+    ref = pl.lanczos_eigs(plan, Lx, kk, split=True)
+    for a, b in zip(res, ref):
+        assert a[2] == b[2]
+        np.testing.assert_allclose(a[0], b[0], rtol=0, atol=1e-12)
+
+
+def test_lanczos_run_gives_up_and_falls_back(cuda, monkeypatch):
+    """A bounded wait that runs out (here after no poll at all) ends the launch; the plan goes
+    back to the launch-per-phase steps and returns their result."""
+    from manifoldem_python_amd import pipeline as pl
+    ns, kk = [300, 120], [9, 7]
+    plan, L = _kernel(cuda, ns, ns)
+    monkeypatch.setattr(pl, "RUN_SPIN", 0)
+    res = pl.lanczos_eigs(plan, L, kk)
+    assert plan._lanczos["run"] is None
+    _check_eigs(plan, L, res, kk)
+
+
+def test_lanczos_run_continues_past_its_lds(cuda, monkeypatch):
+    """A basis that outgrows the workgroups' LDS goes on step by step from the same state."""
+    from manifoldem_python_amd import pipeline as pl
+    made = pl._run_state
+
+    def small(*a):
+        st = made(*a)
+        st["last"] = 16
+        return st
+
+    monkeypatch.setattr(pl, "_run_state", small)
+    ns, kk = [500, 140], [16, 9]
+    plan, L = _kernel(cuda, ns, ns)
+    res = pl.lanczos_eigs(plan, L, kk)
+    assert plan._lanczos["run"] is not None and max(r[2] for r in res) > 16
+    _check_eigs(plan, L, res, kk)

@@ -1,5 +1,6 @@
 """Host-side pieces of the GPU pipeline that need no GPU."""
 import numpy as np
+import pytest
 
 
 def test_lm_ritz_matches_full_decomposition():
@@ -179,3 +180,29 @@ def test_embedd_kept_points_selects_the_surviving_points():
     # -0.0 and 0.0 differ as bit patterns
     got = embedd.kept_points([(-0.0, 1.0), (0.5, 2.0)], [(0.0, 1.0), (0.5, 2.0)])
     np.testing.assert_array_equal(got, [1])
+
+
+@pytest.mark.parametrize("ns,cus", [([1], 256), ([7], 256), ([200], 256), ([4096], 256), ([2000], 64),
+                                    ([2000, 3, 450], 128), ([400] * 64, 256), ([90] * 256, 256)])
+def test_run_groups_cover_the_rows(ns, cus):
+    """Workgroup tables of the Lanczos launches: every row of every PD once, groups consecutive and
+    of at most 64, no more workgroups than CUs, and LDS for RUN_COLUMNS basis columns."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    t = pl.run_groups(ns, np.square(ns), max(ns), cus)
+    assert t is not None and len(t) <= cus
+    for p, n in enumerate(ns):
+        g = t[t[:, 0] == p]
+        assert len(g) <= nat.LANCZOS_RUN_GMAX
+        np.testing.assert_array_equal(g[:, 3], np.arange(len(g)))
+        assert np.all(g[:, 4] == len(g)) and np.all(g[:, 5] == np.nonzero(t[:, 0] == p)[0][0])
+        assert g[0, 1] == 0 and g[-1, 2] == n
+        np.testing.assert_array_equal(g[1:, 1], g[:-1, 2])
+        assert np.all(g[:, 2] > g[:, 1])
+    rows = int((t[:, 2] - t[:, 1]).max())
+    assert 8 * (max(ns) + (pl.RUN_COLUMNS + 4) * rows + pl.RUN_COLUMNS + 1100) <= nat.LANCZOS_RUN_LDS
+
+
+def test_run_groups_refuse_what_does_not_fit():
+    from manifoldem_python_amd import pipeline as pl
+    for ns, cus in (([4097], 256), ([50] * 300, 256), ([2400] * 40, 256), ([2000], 4)):
+        assert pl.run_groups(ns, np.square(ns), max(ns), cus) is None
