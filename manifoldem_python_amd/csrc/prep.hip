@@ -371,19 +371,14 @@ __device__ __forceinline__ void split12(double x, float* hi, float* lo) {
   *lo = (float)(x - h);
 }
 
-// floor and fractional part of hi + lo, hi exact: hi - floor(hi) is exact, adding lo rounds once
+// Integer and fractional part of hi + lo, hi exact, by the floor of their rounded sum: that sum is
+// within 2^-15 of the exact one, so t = (hi - floor) + lo (an exact difference, one rounding) lies
+// in [-2^-15, 1 + 2^-15], where the cubic weights of the neighbouring piece differ from these by
+// the cube of the excess, below 1e-13.
 __device__ __forceinline__ float floor_frac(float hi, float lo, int* fl) {
-  float f0 = floorf(hi);
-  float t = (hi - f0) + lo;
-  if (t < 0.f) {
-    t += 1.f;
-    f0 -= 1.f;
-  } else if (t >= 1.f) {
-    t -= 1.f;
-    f0 += 1.f;
-  }
+  const float f0 = floorf(hi + lo);
   *fl = (int)f0;
-  return t;
+  return (hi - f0) + lo;
 }
 
 template <int NMAX, int NF, int NT>
@@ -424,13 +419,15 @@ __device__ __forceinline__ void spline_sample_inplace(float* buf, int N, int S,
       // |src - h| <= sqrt(2) h for |sin|, |cos| <= 1 (a NaN angle converts to 0), so the first
       // tap lies in [-N, 2N) and one wrap brings it into [0, N); the three after it come from
       // the padding
-      ir -= 1;
-      ic -= 1;
-      ir += ir < 0 ? N : 0;
-      ir -= ir >= N ? N : 0;
-      ic += ic < 0 ? N : 0;
-      ic -= ic >= N ? N : 0;
-      const float* q = buf + __umul24(ir, S) + ic;
+      // (unsigned minima: a negative index is larger than its wrapped value, and an index below
+      // N smaller than itself less N)
+      const unsigned n = N;
+      unsigned jr = (unsigned)ir - 1u, jc = (unsigned)ic - 1u;
+      jr = min(jr, jr + n);
+      jr = min(jr, jr - n);
+      jc = min(jc, jc + n);
+      jc = min(jc, jc - n);
+      const float* q = buf + __umul24(jr, S) + jc;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float* rp = q + u * S;
@@ -682,13 +679,40 @@ __global__ void k_prep_tables(int N, int kind, double Qc, int order, memi_ctf_pa
 }
 
 // NF > 0: a kernel for image side NF only (every size, count and divisor a constant);
-// NF = 0: any side up to NMAX, given at run time.  NT threads per image: 256 where four
-// images fit in one CU's LDS (sides up to 96: four blocks of four waves interleave their
-// barriers and serial spline recursions), else 512.  The 256-thread and the 128 kernels are
-// held to 128 registers: 4 waves per SIMD, i.e. four (two) images per CU, as their LDS allows.
-constexpr int prep_threads(int nmax) { return nmax <= 96 ? 256 : 512; }
-template <int NMAX, int NF, int NT = prep_threads(NMAX)>
-__global__ __launch_bounds__(NT, (NMAX == 128 || NT == 256) ? 4 : 1) void k_prep_images(
+// NF = 0: any side up to NMAX, given at run time.  NT threads per image; see prep_threads.
+//
+// Waves per SIMD the registers are held to: what the images that fit in a CU's LDS can use (side
+// 64: eight images, 96: four, 128: two), short of spilling in the inner loops.  8192 images of
+// 48 x 48: 549 us at six, 605 at four; of 96 x 96 with 512 threads: 1155 us at six, 1342 at five;
+// 2000 of 128 x 128 with 1024 threads: 661 us at eight, 764 at four (512 threads: 687).
+constexpr int prep_waves(int nmax, int nf, int nt) {
+  if (nmax == 160) return nt == 1024 ? 4 : 2;
+  if (nt == 1024) return nf == 128 ? 8 : 4;
+  if (nmax == 128) return 4;
+  if (nt == 512) return nf == 64 ? 8 : nf == 96 ? 6 : 5;
+  return 6;
+}
+
+// Threads per image for n images of side N: enough waves to fill a CU with the images it holds.
+// Few images leave a CU one or two of them, whose serial spline recursions and barriers only
+// more threads shorten (200 images: side 70 77 us with 512 threads, 106 with 256; side 96 91 with
+// 1024, 131 with 256; side 128 147 and 163 with 1024 and 512); with many, more and smaller
+// workgroups overlap better (8192 images: side 70 1020 us with 256, 1161 with 512; side 64 494
+// and 510; but side 96 1242 and 1155, side 128 as above, and side 160, one image per CU, 1131 us
+// per 2000 with 1024 threads against 1399 with 512).
+inline int prep_threads(int N, int64_t n) {
+  constexpr int64_t CUS = 256;
+  if (N > 128) return 1024;
+  if (N == 128) return 1024;
+  if (N > 96) return n <= CUS ? 1024 : 512;
+  if (N == 96) return n <= CUS ? 1024 : 512;
+  if (N == 64) return n <= 4 * CUS ? 512 : 256;
+  return n <= 2 * CUS ? 512 : 256;
+}
+
+template <int NMAX, int NF, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(prep_waves(NMAX, NF, NT))))
+void k_prep_images(
     const float* __restrict__ stack, const int64_t* __restrict__ src,
     const int32_t* __restrict__ conj, const double* __restrict__ rot1,
     const double* __restrict__ rot2, const double* __restrict__ df, int N_arg,
@@ -700,12 +724,15 @@ __global__ __launch_bounds__(NT, (NMAX == 128 || NT == 256) ? 4 : 1) void k_prep
   static_assert(NF == 0 || NF == NMAX, "a fixed-size kernel is sized for its own side");
   const int N = NF > 0 ? NF : N_arg;
   constexpr int BUF = (NMAX + 3) * (NMAX + 3);
-  __shared__ float lds[BUF];
+  __shared__ __attribute__((aligned(16))) float lds[BUF];
   __shared__ cpx tw[NMAX];
   __shared__ int pos[NMAX], rev[NMAX];              // frequency <-> position after the passes
-  __shared__ double red[16];
   float* A = lds;
   const int S = N + 3;
+  // the statistics' partial sums, in the padding rows (filled after the first prefilter): 48
+  // bytes more at side 96 would leave three images per CU instead of four
+  double* red = (double*)(A + ((N * S + 1) & ~1));
+  static_assert(3 * (64 + 3) >= 2 * 32 + 1, "room for 32 doubles in the padding rows");
   const int Nh = N / 2 + 1;
   const int64_t Kh = (int64_t)N * Nh;
   const float* tabf = (const float*)(tab + 2 * Kh);    // filter and envelope (k_prep_tables)
@@ -750,7 +777,7 @@ __global__ __launch_bounds__(NT, (NMAX == 128 || NT == 256) ? 4 : 1) void k_prep
   }
   const double NN = (double)N * N;
   const double mean = block_sum(s1, red) / NN;
-  const double sd = sqrt(block_sum(s2, red + 8) / NN - mean * mean);
+  const double sd = sqrt(block_sum(s2, red + 16) / NN - mean * mean);
   const double inv_sd = 1.0 / sd;
   for (int r = wv; r < N; r += nw)
     for (int c = lane; c < N; c += 64)
@@ -779,9 +806,9 @@ __global__ __launch_bounds__(NT, (NMAX == 128 || NT == 256) ? 4 : 1) void k_prep
   // constant-folded the compiler computes them all ahead and spills
   int n_rt = N;
   asm volatile("" : "+s"(n_rt));
-  spline_sample_inplace<NMAX, 0, NT>(A, n_rt, n_rt + 3, rot1[img]);
+  spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot1[img]);
   bspline_prefilter(A, N, S, zN);
-  spline_sample_inplace<NMAX, 0, NT>(A, n_rt, n_rt + 3, rot2[img]);
+  spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot2[img]);
   if (img_out) {
     float* o = img_out + img * (int64_t)N * N;
     for (int r = wv; r < N; r += nw)
@@ -969,23 +996,33 @@ int memi_prep_images(const float* stack, int64_t n_stack, const int64_t* src,
                      order, *ctf, ws);
   MEMI_CHECK_LAUNCH("k_prep_tables");
   const dim3 g((unsigned)n);
-#define MEMI_PREP(NM, NF)                                                                      \
-  hipLaunchKernelGGL((k_prep_images<NM, NF>), g, dim3(prep_threads(NM)), 0, s, stack, src, conj, \
+#define MEMI_PREP(NM, NF, NT)                                                                    \
+  hipLaunchKernelGGL((k_prep_images<NM, NF, NT>), g, dim3(NT), 0, s, stack, src, conj,           \
                      rot1_deg, rot2_deg, df, N, ws, ctf->ampc, precision, Khp, row0, op_hi,     \
                      op_lo, (float2*)fy, ctf_half, img_out)
+  const int nt = prep_threads(N, n);
   // the power-of-two-rich sides of the standard workloads get their own kernels (a fixed
   // 70 = 2 x 5 x 7 kernel needs more registers than the generic one); any other side runs on
   // the kernel of the next larger size class
   switch (N) {
-    case 64: MEMI_PREP(64, 64); break;
-    case 96: MEMI_PREP(96, 96); break;
-    case 128: MEMI_PREP(128, 128); break;
-    case 160: MEMI_PREP(160, 160); break;
+    case 64:
+      if (nt == 512) MEMI_PREP(64, 64, 512);
+      else MEMI_PREP(64, 64, 256);
+      break;
+    case 96:
+      if (nt == 1024) MEMI_PREP(96, 96, 1024);
+      else MEMI_PREP(96, 96, 512);
+      break;
+    case 128: MEMI_PREP(128, 128, 1024); break;
+    case 160: MEMI_PREP(160, 160, 1024); break;
     default:
-      if (N <= 64) MEMI_PREP(64, 0);
-      else if (N <= 96) MEMI_PREP(96, 0);
-      else if (N <= 128) MEMI_PREP(128, 0);
-      else MEMI_PREP(160, 0);
+      if (N <= 64 && nt == 512) MEMI_PREP(64, 0, 512);
+      else if (N <= 64) MEMI_PREP(64, 0, 256);
+      else if (N <= 96 && nt == 512) MEMI_PREP(96, 0, 512);
+      else if (N <= 96) MEMI_PREP(96, 0, 256);
+      else if (N <= 128 && nt == 1024) MEMI_PREP(128, 0, 1024);
+      else if (N <= 128) MEMI_PREP(128, 0, 512);
+      else MEMI_PREP(160, 0, 1024);
   }
 #undef MEMI_PREP
   MEMI_CHECK_LAUNCH("k_prep_images");

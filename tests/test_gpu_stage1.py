@@ -268,6 +268,21 @@ def _operand_values(op):
             f(op.lo).view(np.float32).astype(np.float64))
 
 
+@pytest.mark.parametrize("n,N", [(512, 48), (513, 48), (1024, 64), (1025, 64), (512, 90), (513, 90),
+                                 (256, 96), (257, 96), (256, 105), (257, 105), (3, 64), (3, 128)])
+def test_fused_prep_thread_counts(cuda, n, N):
+    """memi_prep_images picks its threads per image by side and count: both sides of each line
+    against the staged path, to the float32 bound of test_fused_prep_matches_staged."""
+    s = _setup(n, N, seed=2, conj_frac=0.3)
+    _, a, opa = _gpu_prep(s, cuda, 0, prep="fused")
+    _, b, opb = _gpu_prep(s, cuda, 0, prep="staged")
+    for key in ("imgAll", "fy"):
+        va, vb = a[key].cpu().numpy(), b[key].cpu().numpy()
+        assert np.max(np.abs(va - vb)) < 2e-6 * np.max(np.abs(vb)), key
+    va, vb = _operand_values(opa), _operand_values(opb)
+    assert np.max(np.abs(va - vb)) < 1e-5 * np.max(np.abs(vb))
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("N", [40, 45, 70, 96, 128, 150, 160])
 def test_fused_prep_matches_staged(cuda, precision, N):
