@@ -371,14 +371,14 @@ __device__ __forceinline__ void split12(double x, float* hi, float* lo) {
   *lo = (float)(x - h);
 }
 
-// Integer and fractional part of hi + lo, hi exact, by the floor of their rounded sum: that sum is
-// within 2^-15 of the exact one, so t = (hi - floor) + lo (an exact difference, one rounding) lies
-// in [-2^-15, 1 + 2^-15], where the cubic weights of the neighbouring piece differ from these by
-// the cube of the excess, below 1e-13.
+// floor and fractional part of hi + lo, hi exact: hi - floor(hi) is exact, adding lo rounds once,
+// and the floor of that (-1, 0 or 1) moves both into place
 __device__ __forceinline__ float floor_frac(float hi, float lo, int* fl) {
-  const float f0 = floorf(hi + lo);
-  *fl = (int)f0;
-  return (hi - f0) + lo;
+  const float f0 = floorf(hi);
+  const float t = (hi - f0) + lo;
+  const float d = floorf(t);
+  *fl = (int)(f0 + d);
+  return t - d;
 }
 
 template <int NMAX, int NF, int NT>
@@ -428,10 +428,14 @@ __device__ __forceinline__ void spline_sample_inplace(float* buf, int N, int S,
       jc = min(jc, jc + n);
       jc = min(jc, jc - n);
       const float* q = buf + __umul24(jr, S) + jc;
+      // the order of the products is written out: left to contraction it changes with the code
+      // around it, and with it the last bits of every aligned image
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float* rp = q + u * S;
-        acc += wr[u] * (wc[0] * rp[0] + wc[1] * rp[1] + wc[2] * rp[2] + wc[3] * rp[3]);
+        float row = u == 0 ? fmaf(wc[1], rp[1], wc[0] * rp[0]) : fmaf(wc[0], rp[0], wc[1] * rp[1]);
+        row = fmaf(wc[3], rp[3], fmaf(wc[2], rp[2], row));
+        acc = u == 0 ? wr[0] * row : fmaf(wr[u], row, acc);
       }
       acc *= 1.f / 36.f;          // the two sets of weights were 6x the B-spline's
     }
