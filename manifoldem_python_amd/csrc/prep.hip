@@ -139,16 +139,28 @@ __global__ void k_spectrum_scale(float2* __restrict__ spec, int64_t n, int N, in
     if (i0 + u < n) spec[(i0 + u) * Kh + k] = make_float2(v[u].x * ff, v[u].y * ff);
 }
 
-__global__ void k_mask_multiply(float* __restrict__ img, int64_t total, int N, int disk,
-                                const float* __restrict__ msk2) {
+// A thread per pixel and MASK_IMG images: the mask's value is formed once, and a pixel it leaves as
+// it is (1) is neither read nor written, which is most of a 0 / 1 mask.  Bound by memory: 500 images
+// of 180 x 180 under a volume mask 38 -> 15 us.
+constexpr int MASK_IMG = 8;
+__global__ __launch_bounds__(256) void k_mask_multiply(float* __restrict__ img, int64_t n, int N,
+                                                       int disk,
+                                                       const float* __restrict__ msk2) {
   const int NN = N * N;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int p = (int)(e % NN);
-    float m = 1.f;
-    if (disk && !in_disk(p / N, p % N, N)) m = 0.f;
-    if (msk2) m *= msk2[p];
-    img[e] *= m;
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= NN) return;
+  float m = 1.f;
+  if (disk && !in_disk(p / N, p % N, N)) m = 0.f;
+  if (msk2) m *= msk2[p];
+  if (m == 1.f) return;
+  for (int64_t i0 = blockIdx.y * (int64_t)MASK_IMG; i0 < n; i0 += gridDim.y * (int64_t)MASK_IMG) {
+    float v[MASK_IMG];
+#pragma unroll
+    for (int u = 0; u < MASK_IMG; ++u)
+      if (i0 + u < n) v[u] = img[(i0 + u) * NN + p];
+#pragma unroll
+    for (int u = 0; u < MASK_IMG; ++u)
+      if (i0 + u < n) img[(i0 + u) * NN + p] = v[u] * m;
   }
 }
 
@@ -612,36 +624,87 @@ __global__ void k_phase_flip(const float2* __restrict__ fy, const float* __restr
   }
 }
 
-// thread per half-spectrum bin: loop over images (coalesced across bins)
-__global__ void k_wiener_average(const float2* __restrict__ spec, const float* __restrict__ ctf,
-                                 int64_t n, int64_t Kh, double snr, float2* __restrict__ out) {
-  for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < Kh;
-       k += (int64_t)gridDim.x * blockDim.x) {
+// Sums over the images of one PD, per half-spectrum bin or per pixel.  Bound by memory: each image
+// is read once.  A block takes 64 neighbouring elements (coalesced rows of a wave) and its AVG_WAVES
+// waves take every AVG_WAVES-th image, four loads in flight each, with one float64 reduction over
+// the waves in LDS in wave order: one wave per 64 elements walking all images leaves 250 to 500 waves
+// on the card, each waiting for one load at a time.  500 images of 180 x 180: Wiener sums 192 ->
+// 22 us, moments 128 -> 14.
+constexpr int AVG_WAVES = 16, AVG_UNROLL = 4;
+
+// total over the block's waves of v, for the lane's element: valid in wave 0
+__device__ __forceinline__ double waves_sum(double v, double (*sh)[64]) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __syncthreads();
+  sh[wv][lane] = v;
+  __syncthreads();
+  double t = 0.0;
+  if (wv == 0)
+    for (int w = 0; w < AVG_WAVES; ++w) t += sh[w][lane];
+  return t;
+}
+
+__global__ __launch_bounds__(64 * AVG_WAVES) void k_wiener_average(
+    const float2* __restrict__ spec, const float* __restrict__ ctf, int64_t n, int64_t Kh,
+    double snr, float2* __restrict__ out) {
+  __shared__ double sh[AVG_WAVES][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int64_t k0 = blockIdx.x * (int64_t)64; k0 < Kh; k0 += gridDim.x * (int64_t)64) {
+    const int64_t k = k0 + lane;
     double nr = 0.0, ni = 0.0, den = 0.0;
-    for (int64_t i = 0; i < n; ++i) {
-      const double c = ctf[i * Kh + k];
-      const float2 x = spec[i * Kh + k];
-      nr += x.x * c;
-      ni += x.y * c;
-      den += c * c;
+    for (int64_t i0 = wv; k < Kh && i0 < n; i0 += AVG_WAVES * AVG_UNROLL) {
+      float c[AVG_UNROLL];
+      float2 x[AVG_UNROLL];
+#pragma unroll
+      for (int u = 0; u < AVG_UNROLL; ++u) {
+        const int64_t i = i0 + u * AVG_WAVES;
+        c[u] = i < n ? ctf[i * Kh + k] : 0.f;
+        x[u] = i < n ? spec[i * Kh + k] : make_float2(0.f, 0.f);
+      }
+#pragma unroll
+      for (int u = 0; u < AVG_UNROLL; ++u) {
+        nr += (double)x[u].x * c[u];
+        ni += (double)x[u].y * c[u];
+        den += (double)c[u] * c[u];
+      }
     }
-    const double w = -(den + 1.0 / snr);
-    out[k] = make_float2((float)(nr / w), (float)(ni / w));
+    nr = waves_sum(nr, sh);
+    ni = waves_sum(ni, sh);
+    den = waves_sum(den, sh);
+    if (wv == 0 && k < Kh) {
+      const double w = -(den + 1.0 / snr);
+      out[k] = make_float2((float)(nr / w), (float)(ni / w));
+    }
   }
 }
 
-__global__ void k_image_moments(const float* __restrict__ img, int64_t n, int64_t npix,
-                                double* __restrict__ sum, double* __restrict__ sumsq) {
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < npix;
-       p += (int64_t)gridDim.x * blockDim.x) {
+__global__ __launch_bounds__(64 * AVG_WAVES) void k_image_moments(
+    const float* __restrict__ img, int64_t n, int64_t npix, double* __restrict__ sum,
+    double* __restrict__ sumsq) {
+  __shared__ double sh[AVG_WAVES][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int64_t p0 = blockIdx.x * (int64_t)64; p0 < npix; p0 += gridDim.x * (int64_t)64) {
+    const int64_t p = p0 + lane;
     double s = 0.0, s2 = 0.0;
-    for (int64_t i = 0; i < n; ++i) {
-      const double v = img[i * npix + p];
-      s += v;
-      s2 += v * v;
+    for (int64_t i0 = wv; p < npix && i0 < n; i0 += AVG_WAVES * AVG_UNROLL) {
+      float v[AVG_UNROLL];
+#pragma unroll
+      for (int u = 0; u < AVG_UNROLL; ++u) {
+        const int64_t i = i0 + u * AVG_WAVES;
+        v[u] = i < n ? img[i * npix + p] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < AVG_UNROLL; ++u) {
+        s += (double)v[u];
+        s2 += (double)v[u] * v[u];
+      }
     }
-    sum[p] = s;
-    sumsq[p] = s2;
+    s = waves_sum(s, sh);
+    s2 = waves_sum(s2, sh);
+    if (wv == 0 && p < npix) {
+      sum[p] = s;
+      sumsq[p] = s2;
+    }
   }
 }
 
@@ -926,8 +989,8 @@ int memi_mask_multiply(float* img, int64_t n, int N, int disk, const float* msk2
   MEMI_CHECK_ARG(img && n >= 0 && N > 0, "memi_mask_multiply: bad arguments");
   const int64_t total = n * (int64_t)N * N;
   if (total == 0 || (!disk && !msk2)) return MEMI_OK;
-  hipLaunchKernelGGL(k_mask_multiply, dim3(grid_for(total)), dim3(256), 0, (hipStream_t)stream,
-                     img, total, N, disk, msk2);
+  const dim3 g((unsigned)(((int64_t)N * N + 255) / 256), (unsigned)grid_for(n, MASK_IMG, 65535));
+  hipLaunchKernelGGL(k_mask_multiply, g, dim3(256), 0, (hipStream_t)stream, img, n, N, disk, msk2);
   MEMI_CHECK_LAUNCH("k_mask_multiply");
   return MEMI_OK;
 }
@@ -1088,8 +1151,8 @@ int memi_wiener_average(const void* spec, const float* ctf_half, int64_t n, int 
                         void* out, void* stream) {
   MEMI_CHECK_ARG(spec && ctf_half && out && snr > 0, "memi_wiener_average: bad arguments");
   const int64_t Kh = (int64_t)N * (N / 2 + 1);
-  hipLaunchKernelGGL(k_wiener_average, dim3(grid_for(Kh, 64)), dim3(64), 0, (hipStream_t)stream,
-                     (const float2*)spec, ctf_half, n, Kh, snr, (float2*)out);
+  hipLaunchKernelGGL(k_wiener_average, dim3(grid_for(Kh, 64)), dim3(64 * AVG_WAVES), 0,
+                     (hipStream_t)stream, (const float2*)spec, ctf_half, n, Kh, snr, (float2*)out);
   MEMI_CHECK_LAUNCH("k_wiener_average");
   return MEMI_OK;
 }
@@ -1097,7 +1160,7 @@ int memi_wiener_average(const void* spec, const float* ctf_half, int64_t n, int 
 int memi_image_moments(const float* img, int64_t n, int64_t npix, double* sum, double* sumsq,
                        void* stream) {
   MEMI_CHECK_ARG(img && sum && sumsq && npix > 0, "memi_image_moments: bad arguments");
-  hipLaunchKernelGGL(k_image_moments, dim3(grid_for(npix, 64)), dim3(64), 0,
+  hipLaunchKernelGGL(k_image_moments, dim3(grid_for(npix, 64)), dim3(64 * AVG_WAVES), 0,
                      (hipStream_t)stream, img, n, npix, sum, sumsq);
   MEMI_CHECK_LAUNCH("k_image_moments");
   return MEMI_OK;

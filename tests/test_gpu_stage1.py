@@ -268,6 +268,40 @@ def _operand_values(op):
             f(op.lo).view(np.float32).astype(np.float64))
 
 
+@pytest.mark.parametrize("n,N", [(1, 8), (15, 9), (16, 16), (17, 45), (64, 64), (65, 70), (133, 96)])
+def test_image_sums_and_masks(cuda, n, N):
+    """Per-pixel and per-bin sums over the images and the in-place masks against numpy: float64
+    sums to 64-bit rounding, the Wiener quotient to float32 rounding, masked pixels exactly."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(n * N)
+    Nh = N // 2 + 1
+    x = rng.standard_normal((n, N, N)).astype(np.float32)
+    sp = (rng.standard_normal((n, N, Nh)) + 1j * rng.standard_normal((n, N, Nh))).astype(np.complex64)
+    c = rng.uniform(-1, 1, (n, N * Nh)).astype(np.float32)
+    d = lambda a: torch.as_tensor(a, device=cuda)
+    s = torch.empty(N * N, dtype=torch.float64, device=cuda)
+    s2 = torch.empty_like(s)
+    nat.image_moments(d(x), s, s2)
+    x64 = x.astype(np.float64).reshape(n, -1)
+    np.testing.assert_allclose(s.cpu().numpy(), x64.sum(0), rtol=0,
+                               atol=1e-15 * n * np.abs(x64).max())
+    np.testing.assert_allclose(s2.cpu().numpy(), (x64 ** 2).sum(0), rtol=1e-14 * max(n, 2))
+    out = torch.empty((N, Nh), dtype=torch.complex64, device=cuda)
+    nat.wiener_average(d(sp), d(c), N, 5.0, out)
+    c64 = c.astype(np.float64).reshape(n, N, Nh)
+    want = (sp.astype(np.complex128) * c64).sum(0) / -((c64 ** 2).sum(0) + 1 / 5.0)
+    assert np.max(np.abs(out.cpu().numpy() - want)) < 2 ** -23 * np.max(np.abs(want))
+    m = rng.choice([0.0, 0.25, 1.0, 1.0], (N, N)).astype(np.float32)
+    a = np.arange(N)
+    disk = (2 * a[:, None] - N + 2) ** 2 + (2 * a[None, :] - N) ** 2 < N * N
+    for msk2, on in ((m, False), (None, True), (m, True)):
+        y = d(x)
+        nat.mask_multiply(y, N, disk=on, msk2=None if msk2 is None else d(msk2))
+        want = x * (disk.astype(np.float32) if on else 1) * (1 if msk2 is None else msk2)
+        np.testing.assert_array_equal(y.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("n,N", [(512, 48), (513, 48), (1024, 64), (1025, 64), (512, 90), (513, 90),
                                  (256, 96), (257, 96), (256, 105), (257, 105), (3, 64), (3, 128)])
 def test_fused_prep_thread_counts(cuda, n, N):
