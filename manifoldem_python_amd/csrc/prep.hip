@@ -241,15 +241,16 @@ constexpr int BSPLINE_NT = 16;   // |z|^16 / (1 - |z|) < 1e-9: below float32 rou
 // Cubic B-spline prefilter (the interpolation coefficients of scipy's spline_filter with
 // periodic lines) of every row (ROWS) or column of the image, in place, in float32: the
 // causal recursion c+[k] = x[k] + z c+[k-1] and the anticausal c[k] = z (c[k+1] - c+[k]),
-// times 6.  Each line is cut into nseg segments run by consecutive threads; a segment's first
-// value comes from the truncated periodic sum over the BSPLINE_NT preceding samples (causal)
-// or following coefficients (anticausal), exact to float rounding since |z|^16 < 1e-9.
+// times 6.  Each line is cut into nseg segments of seg_min samples or more, run by consecutive
+// threads; a segment's first value comes from the truncated periodic sum over the BSPLINE_NT
+// preceding samples (causal) or following coefficients (anticausal), exact to float rounding since
+// |z|^16 < 1e-9.
 template <bool ROWS>
-__device__ __forceinline__ void bspline_lines(float* buf, int N, int S, float zN) {
+__device__ __forceinline__ void bspline_lines(float* buf, int N, int S, float zN, int seg_min) {
   const int es = ROWS ? 1 : S;
   const int nt = min(N, BSPLINE_NT);
   const float z = (float)BSPLINE_Z;
-  const int nseg = max(1, min((int)blockDim.x / N, (N + 7) / 8));
+  const int nseg = max(1, min((int)blockDim.x / N, (N + seg_min - 1) / seg_min));
   const int Ls = (N + nseg - 1) / nseg;
   const int t = threadIdx.x;
   const int l = t % N, sg = t / N;              // consecutive threads: consecutive lines
@@ -322,10 +323,11 @@ __device__ __forceinline__ void refresh_pad(float* buf, int N, int S) {
   __syncthreads();
 }
 
-__device__ __forceinline__ void bspline_prefilter(float* buf, int N, int S, float zN) {
-  bspline_lines<true>(buf, N, S, zN);
+__device__ __forceinline__ void bspline_prefilter(float* buf, int N, int S, float zN,
+                                                  int seg_min = 8) {
+  bspline_lines<true>(buf, N, S, zN, seg_min);
   __syncthreads();
-  bspline_lines<false>(buf, N, S, zN);
+  bspline_lines<false>(buf, N, S, zN, seg_min);
   __syncthreads();
   refresh_pad(buf, N, S);
 }
@@ -748,16 +750,18 @@ __global__ void k_prep_tables(int N, int kind, double Qc, int order, memi_ctf_pa
 // NF > 0: a kernel for image side NF only (every size, count and divisor a constant);
 // NF = 0: any side up to NMAX, given at run time.  NT threads per image; see prep_threads.
 //
-// Waves per SIMD the registers are held to: what the images that fit in a CU's LDS can use (side
-// 64: eight images, 96: four, 128: two), short of spilling in the inner loops.  8192 images of
-// 48 x 48: 549 us at six, 605 at four; of 96 x 96 with 512 threads: 1155 us at six, 1342 at five;
-// 2000 of 128 x 128 with 1024 threads: 661 us at eight, 764 at four (512 threads: 687).
+// Waves per SIMD the registers are held to: what the images that fit in a CU's LDS can use (class
+// 64: eight images, 80: five, 96: four, 128 and 136: two), short of spilling in the inner loops.
+// 8192 images of 96 x 96 with 512 threads: 1155 us at six, 1342 at five; of 70 x 70 791 at five,
+// 839 at six; 2000 of 128 x 128 with 1024 threads: 661 us at eight, 764 at four (512 threads:
+// 687); of 135 x 135 820 at eight, two images per CU, 1046 at four, one.
 constexpr int prep_waves(int nmax, int nf, int nt) {
-  if (nmax == 160) return nt == 1024 ? 4 : 2;
-  if (nt == 1024) return nf == 128 ? 8 : 4;
+  if (nmax == 160) return 4;
+  if (nt == 1024) return nf == 128 || nmax == 136 ? 8 : 4;
   if (nmax == 128) return 4;
-  if (nt == 512) return nf == 64 ? 8 : nf == 96 ? 6 : 5;
-  return 6;
+  if (nmax == 112) return 6;
+  if (nt == 512) return nf == 64 ? 8 : 6;
+  return nmax == 80 ? 5 : nmax == 96 ? 4 : 6;
 }
 
 // Threads per image for n images of side N: enough waves to fill a CU with the images it holds.
@@ -766,13 +770,12 @@ constexpr int prep_waves(int nmax, int nf, int nt) {
 // 1024, 131 with 256; side 128 147 and 163 with 1024 and 512); with many, more and smaller
 // workgroups overlap better (8192 images: side 70 1020 us with 256, 1161 with 512; side 64 494
 // and 510; but side 96 1242 and 1155, side 128 as above, and side 160, one image per CU, 1131 us
-// per 2000 with 1024 threads against 1399 with 512).
+// per 2000 with 1024 threads against 1399 with 512).  (Those times are of one build of the kernel
+// with either count; those of the whole kernel now are at the top of fft_lds.h.)
 inline int prep_threads(int N, int64_t n) {
   constexpr int64_t CUS = 256;
-  if (N > 128) return 1024;
-  if (N == 128) return 1024;
-  if (N > 96) return n <= CUS ? 1024 : 512;
-  if (N == 96) return n <= CUS ? 1024 : 512;
+  if (N >= 128) return 1024;
+  if (N >= 96) return n <= CUS ? 1024 : 512;
   if (N == 64) return n <= 4 * CUS ? 512 : 256;
   return n <= 2 * CUS ? 512 : 256;
 }
@@ -799,7 +802,7 @@ void k_prep_images(
   // the statistics' partial sums, in the padding rows (filled after the first prefilter): 48
   // bytes more at side 96 would leave three images per CU instead of four
   double* red = (double*)(A + ((N * S + 1) & ~1));
-  static_assert(3 * (64 + 3) >= 2 * 32 + 1, "room for 32 doubles in the padding rows");
+  static_assert(NMAX >= 64 && 3 * (64 + 3) >= 2 * 32 + 1, "room for 32 doubles in the padding rows");
   const int Nh = N / 2 + 1;
   const int64_t Kh = (int64_t)N * Nh;
   const float* tabf = (const float*)(tab + 2 * Kh);    // filter and envelope (k_prep_tables)
@@ -868,13 +871,16 @@ void k_prep_images(
     }
   __syncthreads();
   const float zN = (float)pow(BSPLINE_Z, (double)N);
-  bspline_prefilter(A, N, S, zN);
+  // segments of the recursions: short chains for small sides (200 images of 48 x 48: 54 us with
+  // 8, 58 with 20 samples at least); the others run as fast with 20, restarting less often
+  const int seg = N <= 80 ? 8 : 20;
+  bspline_prefilter(A, N, S, zN, seg);
   // the rotations run with the side as a run-time value: with every pixel's coordinates
   // constant-folded the compiler computes them all ahead and spills
   int n_rt = N;
   asm volatile("" : "+s"(n_rt));
   spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot1[img]);
-  bspline_prefilter(A, N, S, zN);
+  bspline_prefilter(A, N, S, zN, seg);
   spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot2[img]);
   if (img_out) {
     float* o = img_out + img * (int64_t)N * N;
@@ -1070,7 +1076,9 @@ int memi_prep_images(const float* stack, int64_t n_stack, const int64_t* src,
   const int nt = prep_threads(N, n);
   // the power-of-two-rich sides of the standard workloads get their own kernels (a fixed
   // 70 = 2 x 5 x 7 kernel needs more registers than the generic one); any other side runs on
-  // the kernel of the next larger size class
+  // the kernel of the next larger size class.  The classes between the fixed sides are where one
+  // more image fits in a CU's LDS: 80 (five for four: 8192 images of 70 x 70 879 -> 791 us), 112
+  // (three for two), 136 (two for one: 2000 of 135 x 135 1112 -> 820)
   switch (N) {
     case 64:
       if (nt == 512) MEMI_PREP(64, 64, 512);
@@ -1085,10 +1093,16 @@ int memi_prep_images(const float* stack, int64_t n_stack, const int64_t* src,
     default:
       if (N <= 64 && nt == 512) MEMI_PREP(64, 0, 512);
       else if (N <= 64) MEMI_PREP(64, 0, 256);
+      else if (N <= 80 && nt == 512) MEMI_PREP(80, 0, 512);
+      else if (N <= 80) MEMI_PREP(80, 0, 256);
       else if (N <= 96 && nt == 512) MEMI_PREP(96, 0, 512);
       else if (N <= 96) MEMI_PREP(96, 0, 256);
+      else if (N <= 112 && nt == 1024) MEMI_PREP(112, 0, 1024);
+      else if (N <= 112) MEMI_PREP(112, 0, 512);
       else if (N <= 128 && nt == 1024) MEMI_PREP(128, 0, 1024);
       else if (N <= 128) MEMI_PREP(128, 0, 512);
+      else if (N <= 136 && nt == 1024) MEMI_PREP(136, 0, 1024);
+      else if (N <= 136) MEMI_PREP(136, 0, 512);
       else MEMI_PREP(160, 0, 1024);
   }
 #undef MEMI_PREP

@@ -303,7 +303,9 @@ def test_image_sums_and_masks(cuda, n, N):
 
 
 @pytest.mark.parametrize("n,N", [(512, 48), (513, 48), (1024, 64), (1025, 64), (512, 90), (513, 90),
-                                 (256, 96), (257, 96), (256, 105), (257, 105), (3, 64), (3, 128)])
+                                 (256, 96), (257, 96), (256, 105), (257, 105), (3, 64), (3, 128),
+                                 (4, 80), (600, 80), (5, 81), (4, 112), (300, 112), (5, 120), (6, 135),
+                                 (300, 135), (5, 140), (7, 15), (7, 49), (7, 147)])
 def test_fused_prep_thread_counts(cuda, n, N):
     """memi_prep_images picks its threads per image by side and count: both sides of each line
     against the staged path, to the float32 bound of test_fused_prep_matches_staged."""
