@@ -500,6 +500,15 @@ int memi_kernel_rowsums(const float* D, int n, const double* eps, int n_eps, dou
 int memi_kernel_grad_weights(const float* D, int n, const double* eps, int n_eps,
                              const double* S, const double* g, float* Wt, void* stream);
 
+/* The backward product's right operand, M float32 [n][3][N(N/2+1)] = {C^2, C Re X, C Im X} of the
+ * spectra fy (complex64 [n][N][N/2+1]) and CTFs (float32 [n][N(N/2+1)]), and the gradient from the
+ * product WM = Wt M (the same layout): out = 2 w_k (X WM_0 - C (WM_1 + i WM_2)), complex64 as fy,
+ * w_k the half-spectrum weight (1 or 2) of the bin. */
+int memi_grad_operand(const void* fy, const float* ctf_half, int64_t n, int N, float* M,
+                      void* stream);
+int memi_grad_combine(const void* fy, const float* ctf_half, const float* WM, int64_t n, int N,
+                      void* out, void* stream);
+
 /* ---------------- Optical flow of NLSA movies (CC stage) --------------------------------- */
 /* Movies are float32 [nmov][F][H][W] (frame f of a movie is the reference's
  * np.resize(Mov, (F, dim, dim))[f]).  Arithmetic follows numpy/scipy: float32 where numpy

@@ -99,6 +99,8 @@ _SIGS = {
     "memi_fit1d_tau": [c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp],
     "memi_kernel_rowsums": [c_vp, c_int, c_vp, c_int, c_vp, c_vp, c_vp],
     "memi_kernel_grad_weights": [c_vp, c_int, c_vp, c_int, c_vp, c_vp, c_vp, c_vp],
+    "memi_grad_operand": [c_vp, c_vp, c_i64, c_int, c_vp, c_vp],
+    "memi_grad_combine": [c_vp, c_vp, c_vp, c_i64, c_int, c_vp, c_vp],
     "memi_lanczos_init": [c_vp, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp, c_i64, c_vp],
     "memi_kernel_ell": [c_vp, ctypes.POINTER(PlanInfo), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp],
     "memi_lanczos_steps_sparse": [c_vp, ctypes.POINTER(PlanInfo), c_vp, c_vp, c_vp, c_vp, c_vp,
@@ -936,6 +938,25 @@ def kernel_grad_weights(D, eps, S, g, Wt):
           Wt.dtype == torch.float32 and g.dtype == torch.float64, "kernel_grad_weights: shapes")
     call("memi_kernel_grad_weights", _p(D), D.shape[0], _p(eps), eps.shape[0], _p(S), _p(g),
          _p(Wt), _stream())
+
+
+def grad_operand(fy, ctf_half, N, M):
+    """memi_grad_operand: M (n, 3, N(N/2+1)) = [C^2 | C Re X | C Im X] of each image."""
+    n, Kh = fy.shape[0], N * (N // 2 + 1)
+    _need(fy.dtype == torch.complex64 and fy.numel() == n * Kh and
+          ctf_half.dtype == torch.float32 and ctf_half.numel() >= n * Kh and
+          M.dtype == torch.float32 and M.numel() >= 3 * n * Kh, "grad_operand: shapes")
+    call("memi_grad_operand", _p(fy), _p(ctf_half), n, N, _p(M), _stream())
+
+
+def grad_combine(fy, ctf_half, WM, N, out):
+    """memi_grad_combine: out = 2 w (X WM_0 - C (WM_1 + i WM_2)), complex64 as fy."""
+    n, Kh = fy.shape[0], N * (N // 2 + 1)
+    _need(fy.dtype == torch.complex64 and fy.numel() == n * Kh and
+          ctf_half.dtype == torch.float32 and ctf_half.numel() >= n * Kh and
+          WM.dtype == torch.float32 and WM.numel() >= 3 * n * Kh and
+          out.dtype == torch.complex64 and out.numel() >= n * Kh, "grad_combine: shapes")
+    call("memi_grad_combine", _p(fy), _p(ctf_half), _p(WM), n, N, _p(out), _stream())
 
 
 # --- optical flow of NLSA movies (CC stage) ---------------------------------------------------

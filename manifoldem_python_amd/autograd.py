@@ -12,7 +12,7 @@ K from the stored D instead of storing K:
 
     dL_e/d eps_e   = sum_i T_ei / (2 eps_e^2 S_ei),  S = sum_j K, T = sum_j K D
     Wt_ij          = sum_e g_e (-1/(2 eps_e)) K^e_ij (1/S_ei + 1/S_ej)       (HIP kernel)
-    dL/d conj(X_ik) = w_k [X_ik (Wt B)_ik - C_ik (Wt Y)_ik],  B = C^2, Y = C X  (two GEMMs)
+    dL/d conj(X_ik) = w_k [X_ik (Wt B)_ik - C_ik (Wt Y)_ik],  B = C^2, Y = C X  (one GEMM)
 
 returned in torch's convention for complex inputs (2 dL/d conj X).  The Ferguson log-log slope
 d log sum_ij K / d log eps is ``slope(D, eps)`` below.
@@ -25,21 +25,12 @@ from . import _native as nat
 from . import pipeline as pl
 
 
-def _half_weights(N, device):
-    Nh = N // 2 + 1
-    w = torch.full((Nh,), 2.0, dtype=torch.float32, device=device)
-    w[0] = 1.0
-    if N % 2 == 0:
-        w[-1] = 1.0
-    return w
-
-
 class KernelLogSum(torch.autograd.Function):
     @staticmethod
     def forward(ctx, fy, df, eps, ctf, precision=nat.PREC_FP32):
         dev = fy.device
         n, N, Nh = fy.shape
-        fyd = fy.detach().contiguous()
+        fyd = fy.detach().resolve_conj().contiguous()
         op = pl.Operand(n, N, precision, dev)
         ctf_half = torch.empty((n, N * Nh), dtype=torch.float32, device=dev)
         nat.ctf_pack(fyd, df.detach().contiguous(), N, ctf, precision, op.Khp, 0, op.hi,
@@ -67,17 +58,11 @@ class KernelLogSum(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             Wt = torch.empty((n, n), dtype=torch.float32, device=D.device)
             nat.kernel_grad_weights(D, epsd, S, g, Wt)
-            C = ctf_half.view(n, N, N // 2 + 1)
-            X = fyd
-            B = (C * C).reshape(n, -1)
-            Y = (C * X).reshape(n, -1)
-            WB = (Wt @ B).view_as(C)
-            WYr = (Wt @ Y.real.contiguous()).view_as(C)
-            WYi = (Wt @ Y.imag.contiguous()).view_as(C)
-            w = _half_weights(N, D.device)
-            gr = w * (X.real * WB - C * WYr)
-            gi = w * (X.imag * WB - C * WYi)
-            g_fy = 2.0 * torch.complex(gr, gi)
+            M = torch.empty((n, 3 * N * (N // 2 + 1)), dtype=torch.float32, device=D.device)
+            nat.grad_operand(fyd, ctf_half, N, M)
+            WM = Wt @ M
+            g_fy = torch.empty_like(fyd)
+            nat.grad_combine(fyd, ctf_half, WM, N, g_fy)
         return g_fy, None, g_eps, None, None
 
 

@@ -88,3 +88,71 @@ def test_backward_matches_float64_autograd_and_fd(cuda, n, N):
         fd = float(((_ref_loss(xp, C64, w, e.detach())[0] - _ref_loss(xm, C64, w, e.detach())[0])
                     * g.cpu()).sum()) / (2 * h)
         assert abs(fd - gxr[i, a, b]) <= 1e-4 * max(1.0, np.max(np.abs(gxr)))
+
+
+@pytest.mark.parametrize("n,ne", [(1, 1), (31, 16), (32, 17), (33, 41), (65, 3), (100, 32)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_kernel_grad_weights_tiles(cuda, n, ne, symmetric):
+    """memi_kernel_grad_weights at tile edges and eps counts around a round, for a symmetric D (one
+    exponential for both entries) and any other, against float64: to float32 rounding."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(n + ne)
+    D = rng.uniform(0, 4, (n, n)).astype(np.float32)
+    if symmetric:
+        D = np.triu(D, 1) + np.triu(D, 1).T
+    eps, S = rng.uniform(0.5, 2, ne), rng.uniform(1, 2, (ne, n))
+    g = rng.standard_normal(ne)
+    d = lambda a: torch.as_tensor(a, device=cuda)
+    Wt = torch.empty((n, n), dtype=torch.float32, device=cuda)
+    nat.kernel_grad_weights(d(D), d(eps), d(S), d(g), Wt)
+    c = 1 / (2 * eps)[:, None, None]
+    t = -g[:, None, None] * c * np.exp(-D.astype(np.float64) * c) * (1 / S[:, :, None] + 1 / S[:, None, :])
+    want = t.sum(0)
+    np.fill_diagonal(want, 0)
+    assert np.max(np.abs(Wt.cpu().numpy() - want)) <= 2 ** -23 * max(np.max(np.abs(want)), 1e-30)
+
+
+@pytest.mark.parametrize("n,N", [(1, 8), (3, 9), (5, 45), (2, 64)])
+def test_gradient_operand_and_combination(cuda, n, N):
+    """memi_grad_operand to the bit and memi_grad_combine to float32 rounding against numpy, at odd
+    and even sides (the half-spectrum weights of the first and last column)."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(n * N)
+    Nh = N // 2 + 1
+    X = (rng.standard_normal((n, N, Nh)) + 1j * rng.standard_normal((n, N, Nh))).astype(np.complex64)
+    C = rng.uniform(-1, 1, (n, N, Nh)).astype(np.float32)
+    WM = rng.standard_normal((n, 3, N, Nh)).astype(np.float32)
+    d = lambda a: torch.as_tensor(a, device=cuda)
+    M = torch.empty((n, 3, N, Nh), dtype=torch.float32, device=cuda)
+    nat.grad_operand(d(X), d(C), N, M)
+    np.testing.assert_array_equal(M.cpu().numpy(), np.stack([C * C, C * X.real, C * X.imag], 1))
+    out = torch.empty((n, N, Nh), dtype=torch.complex64, device=cuda)
+    nat.grad_combine(d(X), d(C), d(WM), N, out)
+    w = np.full(Nh, 2.0)
+    w[0] = 1.0
+    if N % 2 == 0:
+        w[-1] = 1.0
+    W = WM.astype(np.float64)
+    want = 2 * w * (X.astype(np.complex128) * W[:, 0] - C * (W[:, 1] + 1j * W[:, 2]))
+    assert np.max(np.abs(out.cpu().numpy() - want)) < 4 * 2 ** -24 * np.max(np.abs(want))
+
+
+def test_logsum_gradient_of_a_conjugate_view(cuda):
+    """Images given as a lazily conjugated view: the same gradient as for the copy."""
+    import torch
+    from manifoldem_python_amd import _native as nat, autograd, synth
+    rng = np.random.default_rng(3)
+    base = torch.fft.rfft2(torch.as_tensor(rng.standard_normal((20, 16, 16)).astype(np.float32),
+                                           device=cuda))
+    df = torch.as_tensor(rng.uniform(5e3, 3e4, 20), device=cuda)
+    ctf = nat.ctf_params(synth.PIX, synth.CS, synth.EKV, synth.AMPC, np.inf)
+    eps = torch.tensor([2e3, 8e3], dtype=torch.float64, device=cuda)
+    grads = []
+    for lazy in (True, False):
+        x = base.clone().requires_grad_(True)
+        y = x.conj() if lazy else x.conj().resolve_conj()
+        autograd.kernel_logsum(y, df, eps, ctf).sum().backward()
+        grads.append(x.grad.resolve_conj().cpu().numpy())
+    np.testing.assert_array_equal(grads[0], grads[1])
