@@ -246,11 +246,12 @@ constexpr int BSPLINE_NT = 16;   // |z|^16 / (1 - |z|) < 1e-9: below float32 rou
 // preceding samples (causal) or following coefficients (anticausal), exact to float rounding since
 // |z|^16 < 1e-9.
 template <bool ROWS>
-__device__ __forceinline__ void bspline_lines(float* buf, int N, int S, float zN, int seg_min) {
+__device__ __forceinline__ void bspline_lines(float* buf, int N, int S, float zN, int seg_min,
+                                              int threads) {
   const int es = ROWS ? 1 : S;
   const int nt = min(N, BSPLINE_NT);
   const float z = (float)BSPLINE_Z;
-  const int nseg = max(1, min((int)blockDim.x / N, (N + seg_min - 1) / seg_min));
+  const int nseg = max(1, min(threads / N, (N + seg_min - 1) / seg_min));
   const int Ls = (N + nseg - 1) / nseg;
   const int t = threadIdx.x;
   const int l = t % N, sg = t / N;              // consecutive threads: consecutive lines
@@ -324,10 +325,10 @@ __device__ __forceinline__ void refresh_pad(float* buf, int N, int S) {
 }
 
 __device__ __forceinline__ void bspline_prefilter(float* buf, int N, int S, float zN,
-                                                  int seg_min = 8) {
-  bspline_lines<true>(buf, N, S, zN, seg_min);
+                                                  int seg_min = 8, int threads = blockDim.x) {
+  bspline_lines<true>(buf, N, S, zN, seg_min, threads);
   __syncthreads();
-  bspline_lines<false>(buf, N, S, zN, seg_min);
+  bspline_lines<false>(buf, N, S, zN, seg_min, threads);
   __syncthreads();
   refresh_pad(buf, N, S);
 }
@@ -336,6 +337,28 @@ __device__ __forceinline__ void bspline_prefilter(float* buf, int N, int S, floa
 // angle_deg into dst (row stride ds).  Source rows/columns are clamped to [-N+2, 2N-3] before
 // the taps, which changes nothing for finite angles (|src - h| <= sqrt(2) h) and, with one
 // wrap of the first tap into [0, N), keeps all four taps inside the padded image.
+__device__ __forceinline__ float spline_pixel(const float* src, int N, int S, double sr, double sc,
+                                              double lo, double hi) {
+  const double fr = floor(sr), fc = floor(sc);
+  float wr[4], wc[4];
+  bspline_w((float)(sr - fr), wr);
+  bspline_w((float)(sc - fc), wc);
+  int ir = (int)fmin(fmax(fr, lo), hi) - 1;
+  int ic = (int)fmin(fmax(fc, lo), hi) - 1;
+  ir += ir < 0 ? N : 0;
+  ir -= ir >= N ? N : 0;
+  ic += ic < 0 ? N : 0;
+  ic -= ic >= N ? N : 0;
+  const float* p = src + ir * S + ic;
+  float acc = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float* rp = p + q * S;
+    acc += wr[q] * (wc[0] * rp[0] + wc[1] * rp[1] + wc[2] * rp[2] + wc[3] * rp[3]);
+  }
+  return acc;
+}
+
 __device__ inline void spline_sample(const float* src, int N, int S, double angle_deg, float* dst,
                                      int ds) {
   double sn, cs;
@@ -348,28 +371,46 @@ __device__ inline void spline_sample(const float* src, int N, int S, double angl
     const double br = h + cs * dr, bc = h - sn * dr;
     for (int c = lane; c < N; c += 64) {
       const double dc = c - h;
-      const double sr = br + sn * dc;
-      const double sc = bc + cs * dc;
-      const double fr = floor(sr), fc = floor(sc);
-      float wr[4], wc[4];
-      bspline_w((float)(sr - fr), wr);
-      bspline_w((float)(sc - fc), wc);
-      int ir = (int)fmin(fmax(fr, lo), hi) - 1;
-      int ic = (int)fmin(fmax(fc, lo), hi) - 1;
-      ir += ir < 0 ? N : 0;
-      ir -= ir >= N ? N : 0;
-      ic += ic < 0 ? N : 0;
-      ic -= ic >= N ? N : 0;
-      const float* p = src + ir * S + ic;
-      float acc = 0.f;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float* rp = p + q * S;
-        acc += wr[q] * (wc[0] * rp[0] + wc[1] * rp[1] + wc[2] * rp[2] + wc[3] * rp[3]);
-      }
-      dst[r * ds + c] = acc;
+      dst[r * ds + c] = spline_pixel(src, N, S, br + sn * dc, bc + cs * dc, lo, hi);
     }
   }
+}
+
+// the same over the image itself: every pixel into registers, a barrier, then the stores
+template <int NMAX, int NT>
+__device__ __forceinline__ void spline_sample_over(float* buf, int N, int S, double angle_deg) {
+  constexpr int ROWS = (NMAX * 64 + NT - 1) / NT, COLS = (NMAX + 63) / 64;
+  double sn, cs;
+  sincospi(angle_deg / 180.0, &sn, &cs);
+  const double h = 0.5 * (N - 1);
+  const double lo = 2 - N, hi = 2 * N - 3;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  float v[ROWS][COLS];
+#pragma unroll
+  for (int a = 0; a < ROWS; ++a) {
+    const int r = wv + a * (NT / 64);
+    const double dr = r - h;
+    const double br = h + cs * dr, bc = h - sn * dr;
+#pragma unroll
+    for (int b = 0; b < COLS; ++b) {
+      const int c = lane + 64 * b;
+      const double dc = c - h;
+      v[a][b] = 0.f;
+      if (r < N && c < N) v[a][b] = spline_pixel(buf, N, S, br + sn * dc, bc + cs * dc, lo, hi);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < ROWS; ++a) {
+    const int r = wv + a * (NT / 64);
+#pragma unroll
+    for (int b = 0; b < COLS; ++b) {
+      const int c = lane + 64 * b;
+      if (r < N && c < N) buf[r * S + c] = v[a][b];
+    }
+  }
+  __syncthreads();
 }
 
 // spline_sample into the same LDS image: thread t evaluates pixels p = t + NT k (row p / N,
@@ -469,14 +510,17 @@ __device__ __forceinline__ void spline_sample_inplace(float* buf, int N, int S,
   __syncthreads();
 }
 
-// One block of 512 threads per image, the image (row stride N + 3, padded) in LDS.
-// NBUF = 2: mask, rotate by ang1 in place, rotate by ang2 into out.  NBUF = 1: (mask if disk,)
-// rotate by ang1 into out; the host runs it twice.  in and out may be the same buffer (each
-// block reads its whole image before writing).
-template <int NMAX, int NBUF>
-__global__ __launch_bounds__(512) void k_align_images(const float* in, const double* ang1,
-                                                      const double* ang2, int N, int disk,
-                                                      float* out) {
+// One block of NT threads per image, the image (row stride N + 3, padded) in LDS: mask, rotate by
+// ang1 in place, rotate by ang2 into out.  in and out may be the same buffer (each block reads its
+// whole image before writing).  Sides above 140 leave a CU one image, which gets 1024 threads and
+// stays in LDS between the rotations; their recursions keep the segments of 512 threads and their
+// first rotation its float64 coordinates, so the result does not depend on the thread count.
+// Bound by the sampling's float64 coordinates and 16 taps.  500 images of 180 x 180: 264 us,
+// 316 as two launches of 512 threads.
+template <int NMAX, int NT>
+__global__ __launch_bounds__(NT) void k_align_images(const float* in, const double* ang1,
+                                                     const double* ang2, int N, int disk,
+                                                     float* out) {
   __shared__ float lds[(NMAX + 3) * (NMAX + 3)];
   const int S = N + 3;
   const int64_t img = blockIdx.x;
@@ -494,15 +538,13 @@ __global__ __launch_bounds__(512) void k_align_images(const float* in, const dou
     }
   __syncthreads();
   const float zN = (float)pow(BSPLINE_Z, (double)N);
-  bspline_prefilter(A, N, S, zN);
-  float* o = out + img * N * N;
-  if constexpr (NBUF == 2) {
+  bspline_prefilter(A, N, S, zN, 8, 512);
+  if constexpr (NT == 512)
     spline_sample_inplace<NMAX, 0, 512>(A, N, S, ang1[img]);
-    bspline_prefilter(A, N, S, zN);
-    spline_sample(A, N, S, ang2[img], o, N);
-  } else {
-    spline_sample(A, N, S, ang1[img], o, N);
-  }
+  else
+    spline_sample_over<NMAX, NT>(A, N, S, ang1[img]);
+  bspline_prefilter(A, N, S, zN, 8, 512);
+  spline_sample(A, N, S, ang2[img], out + img * N * N, N);
 }
 
 __device__ inline uint16_t bf16_rne(float f) {
@@ -1023,19 +1065,16 @@ int memi_align_images(const float* in, const double* rot1_deg, const double* rot
   MEMI_CHECK_ARG(n < ((int64_t)1 << 31), "memi_align_images: too many images");
   hipStream_t s = (hipStream_t)stream;
   const dim3 g((unsigned)n), b(512);
-  if (N <= 64) {
-    hipLaunchKernelGGL((k_align_images<64, 2>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk, out);
-  } else if (N <= 96) {          // 39 KB of LDS: four blocks per CU
-    hipLaunchKernelGGL((k_align_images<96, 2>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk, out);
-  } else if (N <= 140) {
-    hipLaunchKernelGGL((k_align_images<140, 2>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk, out);
-  } else {
-    hipLaunchKernelGGL((k_align_images<MEMI_ALIGN_MAX_N, 1>), g, b, 0, s, in, rot1_deg, rot2_deg,
-                       N, disk, out);
-    MEMI_CHECK_LAUNCH("k_align_images");
-    hipLaunchKernelGGL((k_align_images<MEMI_ALIGN_MAX_N, 1>), g, b, 0, s, out, rot2_deg, rot2_deg,
-                       N, 0, out);
-  }
+  if (N <= 64)
+    hipLaunchKernelGGL((k_align_images<64, 512>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk, out);
+  else if (N <= 96)              // 39 KB of LDS: four blocks per CU
+    hipLaunchKernelGGL((k_align_images<96, 512>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk, out);
+  else if (N <= 140)
+    hipLaunchKernelGGL((k_align_images<140, 512>), g, b, 0, s, in, rot1_deg, rot2_deg, N, disk,
+                       out);
+  else
+    hipLaunchKernelGGL((k_align_images<MEMI_ALIGN_MAX_N, 1024>), g, dim3(1024), 0, s, in, rot1_deg,
+                       rot2_deg, N, disk, out);
   MEMI_CHECK_LAUNCH("k_align_images");
   return MEMI_OK;
 }

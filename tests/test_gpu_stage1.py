@@ -91,6 +91,28 @@ def test_spline_rotate_matches_ndimage(cuda, N):
     assert err < 2e-6, err
 
 
+@pytest.mark.parametrize("N", [140, 141, 170, 171, 195, 196])
+def test_fused_alignment_at_class_edges(cuda, N):
+    """memi_align_images on both sides of its thread-count line and at the largest side: against
+    the oracle's two rotations, to the bound of test_fused_alignment_matches_ndimage, and in place
+    to the same bits."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    from oracle import distance as od
+    rng = np.random.default_rng(N)
+    img = rng.normal(size=(2, N, N))
+    a1, a2 = rng.uniform(-360, 360, 2), rng.uniform(0, 360, 2)
+    msk = od.annular_mask(0, N / 2.0, N, N)
+    ref = np.stack([od.rotatefill(od.rotatefill(img[i] * msk, a1[i]), a2[i]) for i in range(2)])
+    y = torch.as_tensor(img, dtype=torch.float32, device=cuda)
+    out = torch.empty_like(y)
+    t1, t2 = torch.as_tensor(a1, device=cuda), torch.as_tensor(a2, device=cuda)
+    nat.align_images(y, t1, t2, N, out, disk=True)
+    assert np.max(np.abs(out.cpu().numpy() - ref)) < 3e-6 * np.max(np.abs(ref))
+    nat.align_images(y, t1, t2, N, y, disk=True)
+    assert torch.equal(y, out)
+
+
 @pytest.mark.parametrize("N", [40, 45, 96, 128, 160])
 def test_fused_alignment_matches_ndimage(cuda, N):
     """memi_align_images (disk mask, then two rotations, recursive B-spline prefilter in LDS)
