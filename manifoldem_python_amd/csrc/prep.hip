@@ -532,10 +532,11 @@ __device__ __forceinline__ void spline_sample_inplace(float* buf, int N, int S,
 // whole image before writing).  Sides above 140 leave a CU one image, which gets 1024 threads and
 // stays in LDS between the rotations; their recursions keep the segments of 512 threads and their
 // first rotation its float64 coordinates, so the result does not depend on the thread count.
-// Bound by the sampling's float64 coordinates and 16 taps.  500 images of 180 x 180: 264 us,
-// 316 as two launches of 512 threads.
+// Bound by the sampling's float64 coordinates and 16 taps.  2000 images of 180 x 180: 809 us, 1258
+// as two launches of 512 threads; 500: 252 and 316.  Registers are held to four waves per SIMD: one
+// more (129) leaves side 140 one image per CU instead of two (500 of 128 x 128: 154 us for 126).
 template <int NMAX, int NT>
-__global__ __launch_bounds__(NT) void k_align_images(const float* in, const double* ang1,
+__global__ __launch_bounds__(NT, 4) void k_align_images(const float* in, const double* ang1,
                                                      const double* ang2, int N, int disk,
                                                      float* out) {
   __shared__ float lds[(NMAX + 3) * (NMAX + 3)];
@@ -544,15 +545,25 @@ __global__ __launch_bounds__(NT) void k_align_images(const float* in, const doub
   const float* src = in + img * N * N;
   float* A = lds;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int r = wv; r < N; r += nw)
-    for (int c = lane; c < N; c += 64) {
-      float v = src[r * N + c];
-      if (disk) {
-        const int xd = 2 * r - N + 2, yd = 2 * c - N;     // annularMask.op(0, N/2, N, N)
-        if (xd * xd + yd * yd >= N * N) v = 0.f;
+  constexpr int RB = 4, CB = (NMAX + 63) / 64;    // four rows' loads in flight per wave
+  for (int r0 = wv; r0 < N; r0 += RB * nw) {
+    float v[RB][CB];
+#pragma unroll
+    for (int u = 0; u < RB; ++u)
+#pragma unroll
+      for (int k = 0; k < CB; ++k) {
+        const int r = r0 + u * nw, c = lane + 64 * k;
+        v[u][k] = r < N && c < N ? src[r * N + c] : 0.f;
       }
-      A[r * S + c] = v;
-    }
+#pragma unroll
+    for (int u = 0; u < RB; ++u)
+#pragma unroll
+      for (int k = 0; k < CB; ++k) {
+        const int r = r0 + u * nw, c = lane + 64 * k;
+        const int xd = 2 * r - N + 2, yd = 2 * c - N;       // annularMask.op(0, N/2, N, N)
+        if (r < N && c < N) A[r * S + c] = disk && xd * xd + yd * yd >= N * N ? 0.f : v[u][k];
+      }
+  }
   __syncthreads();
   const float zN = (float)pow(BSPLINE_Z, (double)N);
   bspline_prefilter(A, N, S, zN, 8, 512);
