@@ -597,9 +597,13 @@ __global__ void k_fer_thr_copy(int64_t npd, const double* __restrict__ st,
   }
 }
 
-// FM_LANES threads per eps: the series over the buckets below the eps's cut, every FM_LANES-th of
-// them each (one thread per eps walks up to 544 dependent series: one PD of 1273, 1501 eps 73 us
-// with one, 10 us with eight)
+// FM_LANES threads per eps evaluate the series of as many neighbouring buckets below the eps's cut;
+// two of them then add the terms to the sums one after another in bucket order, each by an fma from
+// LDS.  The sums therefore do not depend on FM_LANES, to the last bit: the tanh fit of the log sums
+// can cross a plateau where its step is rounding noise, and one unit in the last place of a log sum
+// moves some bandwidths by 1e-6 there.  (The counts are whole numbers, exact in any order.)  Bound by
+the latency of a round's moments and of the chain: one PD of 1273, 1501 eps 12 us, 73 with one
+thread per eps; 64 PDs of about 400 40 us.
 constexpr int FM_LANES = 8;
 
 __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restrict__ logEps,
@@ -608,6 +612,7 @@ __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restr
                                                            const double* __restrict__ M,
                                                            double* __restrict__ out) {
   __shared__ double cen[FM_BMAX], hw[FM_BMAX];
+  __shared__ double term[3][256];
   const int pd = blockIdx.y;
   const double* g = gp + FM_GP * (int64_t)pd;
   const double w = g[1], base = g[2];
@@ -636,33 +641,47 @@ __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restr
   const double c = 1.0 / (2.0 * exp(logEps[e]));
   const int jmax = min(B, max(0, e * s - b0));
   const double* Mp = M + (int64_t)pd * FM_BMAX * FM_NM;
-  double S = 0.0, SX = 0.0, CN = 0.0;
-  for (int k = lane; k < jmax; k += FM_LANES) {
-    const double xb = cen[k] * c;
-    if (xb > 800.0) break;                            // later buckets underflow too
-    const double t = -hw[k] * c;
-    const double* m = Mp + (int64_t)k * FM_NM;
-    double s0 = m[FM_NM - 2] * invf[FM_NM - 2], s1 = m[FM_NM - 1] * invf[FM_NM - 2];
-    for (int q = FM_NM - 3; q >= 0; --q) {
-      s0 = s0 * t + m[q] * invf[q];
-      s1 = s1 * t + m[q + 1] * invf[q];
+  double* te = &term[0][threadIdx.x - lane];
+  double* tf = &term[lane == 1 ? 2 : 1][threadIdx.x - lane];
+  double acc = lane == 1 ? 0.0 : zeros;               // lane 0: S, lane 1: SX
+  double CN = 0.0;
+  for (int k0 = 0; k0 < jmax; k0 += FM_LANES) {
+    if (cen[k0] * c > 800.0) break;                   // later buckets underflow too
+    const int k = k0 + lane;
+    double ex = 0.0, s0 = 0.0, g1 = 0.0;              // a bucket past the last one adds zero
+    const double xb = k < jmax ? cen[k] * c : INFINITY;
+    if (!(xb > 800.0)) {
+      const double t = -hw[k] * c;
+      const double* m = Mp + (int64_t)k * FM_NM;
+      double s1 = m[FM_NM - 1] * invf[FM_NM - 2];
+      s0 = m[FM_NM - 2] * invf[FM_NM - 2];
+      for (int q = FM_NM - 3; q >= 0; --q) {
+        s0 = fma(s0, t, m[q] * invf[q]);
+        s1 = fma(s1, t, m[q + 1] * invf[q]);
+      }
+      ex = exp(-xb);
+      g1 = fma(xb, s0, -(t * s1));
+      CN += m[0];
     }
-    const double ex = exp(-xb);
-    S += ex * s0;
-    SX += ex * (xb * s0 - t * s1);
-    CN += m[0];
+    term[0][threadIdx.x] = ex;
+    term[1][threadIdx.x] = s0;
+    term[2][threadIdx.x] = g1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    double p[FM_LANES], f[FM_LANES];
+#pragma unroll
+    for (int j = 0; j < FM_LANES; ++j) {
+      p[j] = te[j];
+      f[j] = tf[j];
+    }
+#pragma unroll
+    for (int j = 0; j < FM_LANES; ++j) acc = fma(p[j], f[j], acc);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
 #pragma unroll
-  for (int off = 1; off < FM_LANES; off *= 2) {
-    S += __shfl_xor(S, off, 64);
-    SX += __shfl_xor(SX, off, 64);
-    CN += __shfl_xor(CN, off, 64);
-  }
-  if (lane != 0) return;
+  for (int off = 1; off < FM_LANES; off *= 2) CN += __shfl_xor(CN, off, 64);
   double* o = out + ((int64_t)pd * n_eps + e) * 3;
-  o[0] = S + zeros;
-  o[1] = SX;
-  o[2] = CN + zeros;
+  if (lane < 2) o[lane] = acc;
+  if (lane == 0) o[2] = CN + zeros;
 }
 
 // ------------------------------------------------------------------ normalisation ------

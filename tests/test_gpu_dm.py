@@ -430,6 +430,61 @@ def test_ferguson_sweeps_cut_into_parts(cuda, n, k, n_eps):
             assert abs(S[m][0][0, e] - ref) <= tol * ref, (m, e)
 
 
+def test_ferguson_series_sums_keep_the_bucket_order(cuda):
+    """The moment series' sums equal, bit for bit, one chain over the buckets in order starting from
+    the zero entries, each term added by an fma: the bandwidth fit magnifies a last bit of a log
+    sum up to 1e-6 when it crosses a plateau.  The chain is formed here from the moments and grid
+    parameters the call leaves in its workspace, with the device's exp and libm's fma."""
+    import ctypes
+    import ctypes.util
+    import math
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    fma = ctypes.CDLL(ctypes.util.find_library("m")).fma
+    fma.restype, fma.argtypes = ctypes.c_double, [ctypes.c_double] * 3
+    exp = lambda a: torch.exp(torch.as_tensor(np.asarray(a, dtype=np.float64),
+                                              device=cuda)).cpu().numpy()
+    ns, ks = [150, 400, 90], [150, 60, 30]
+    D = [_distance_matrix(n, 40 + i) for i, n in enumerate(ns)]
+    D[1][5, 6] = D[1][6, 5] = 0.0                     # zero entries
+    plan = nat.Plan(np.concatenate(([0], np.cumsum(ns)[:-1])), ns, ks, chunks=1)
+    flat = torch.as_tensor(np.concatenate([d.astype(np.float32).ravel() for d in D]), device=cuda)
+    mask = pl.knn_mask(plan, flat)
+    le = pl.LOG_EPS
+    npd, n_eps = len(ns), len(le)
+    le0, dle = pl.uniform_grid(le)
+    out = torch.empty(npd * (3 * n_eps + 2), dtype=torch.float64, device=cuda)
+    ws = torch.empty(npd * nat.FM_WS_PER_PD, dtype=torch.float64, device=cuda)
+    nat.ferguson_moments(plan, flat, mask, torch.as_tensor(le, device=cuda), le0, dle, out, ws)
+    got = out[:npd * n_eps * 3].cpu().numpy().reshape(npd, n_eps, 3)
+    ws = ws.cpu().numpy()
+    gp = ws[6 * npd:14 * npd].reshape(npd, 8)
+    M = ws[14 * npd:].reshape(npd, -1, 18)
+    inv = [1.0 / math.factorial(q) for q in range(17)]
+    for p in range(npd):
+        _, w, base, b0, B, s, zeros, direct = gp[p]
+        b0, B, s = int(b0), int(B), int(s)
+        assert not direct and B > 20
+        edge = exp([fma(float(b0 + k), w, base) for k in range(B + 1)])
+        cen, hw = 0.5 * (edge[:-1] + edge[1:]), 0.5 * (edge[1:] - edge[:-1])
+        inside = [e for e in range(n_eps) if 0 < min(B, e * s - b0)]
+        for e in inside[::max(1, len(inside) // 25)]:
+            c = 1.0 / (2.0 * exp(le[e:e + 1])[0])
+            ex = exp(-(cen * c))
+            S, SX, CN = zeros, 0.0, zeros
+            for k in range(min(B, max(0, e * s - b0))):
+                xb, t, m = cen[k] * c, -hw[k] * c, M[p, k]
+                if xb > 800.0:
+                    break
+                s0, s1 = m[16] * inv[16], m[17] * inv[16]
+                for q in range(15, -1, -1):
+                    s0, s1 = fma(s0, t, m[q] * inv[q]), fma(s1, t, m[q + 1] * inv[q])
+                S = fma(ex[k], s0, S)
+                SX = fma(ex[k], fma(xb, s0, -(t * s1)), SX)
+                CN += m[0]
+            assert (S, SX, CN) == tuple(got[p, e]), (p, e)
+
+
 @pytest.mark.parametrize("split", [True, False])
 def test_batched_lanczos_many_pds(cuda, split):
     """80 PDs of 40-160 points: the many-PD orthogonalisation (waves walking the live
