@@ -602,8 +602,8 @@ __global__ void k_fer_thr_copy(int64_t npd, const double* __restrict__ st,
 // LDS.  The sums therefore do not depend on FM_LANES, to the last bit: the tanh fit of the log sums
 // can cross a plateau where its step is rounding noise, and one unit in the last place of a log sum
 // moves some bandwidths by 1e-6 there.  (The counts are whole numbers, exact in any order.)  Bound by
-the latency of a round's moments and of the chain: one PD of 1273, 1501 eps 12 us, 73 with one
-thread per eps; 64 PDs of about 400 40 us.
+// the latency of a round's moments and of the chain: one PD of 1273, 1501 eps 12 us, 73 with one
+// thread per eps; 64 PDs of about 400 40 us.
 constexpr int FM_LANES = 8;
 
 __global__ __launch_bounds__(256) void k_fer_sweep_moments(const double* __restrict__ logEps,
