@@ -1,6 +1,7 @@
 // Stage 3 NLSA kernels.  Reference: NLSA.py:23-158, get_wiener.py:9-21, svdRF.py:9-35,
 // L2_distance.py:8-41, psiAnalysisParS2.py:89-90.
 #include "common.h"
+#include <type_traits>
 
 namespace memi {
 
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(512) void k_supervectors(
   const int m = n - C;
   const int i0 = (lane >> kshift) * steps;                       // this lane's steps
   // element offsets (OFF: 32 bits when they fit, one register per address); images outside the
-  // steps' range are read at its ends and weigh zero
+  // steps' range are read at its ends and enter no sum
   auto img = [&](int j) { return (OFF)min(max(j, 0), n - 2) * (OFF)Kh + (OFF)kc; };
   auto ctf_at = [&](int t) { return ctf[(OFF)min(t, n - 1) * (OFF)Kh + (OFF)kc]; };
   double W = 1.0 / snr;
@@ -144,8 +145,13 @@ __global__ __launch_bounds__(512) void k_supervectors(
   window(0);
   __syncthreads();
   weights(us[0], mus[0]);
+  // Steps past a piece's end take zero for the images too: their weights are zero, but the history
+  // holds images of other delays' sums, which need not be finite.  Only the rounds that reach past
+  // an end (TAIL) pay for it.
+  const int lim = min(steps, m - i0);
+  const int full = min(steps, m - (pieces - 1) * steps);
   int b = 0;
-  for (int c0 = 0; c0 < steps; c0 += SG) {
+  auto round = [&](auto TAIL, int c0) __attribute__((always_inline)) {
     __syncthreads();       // this round's weights are in us[b], the next one's mu in mus[b ^ 1]
     stage_mu(c0 + 2 * SG, mus[b]);
     if (g0 >= C) window(c0 + SG);            // a wave with no delays left only computes weights
@@ -163,7 +169,8 @@ __global__ __launch_bounds__(512) void k_supervectors(
         if (t + 1 < SG) un = us[b][t + 1][half][lane];
 #pragma unroll
         for (int d = 0; d < SG; ++d) {
-          const float2 g = t >= d ? cur[t >= d ? t - d : 0] : prev[t >= d ? 0 : SG + t - d];
+          float2 g = t >= d ? cur[t >= d ? t - d : 0] : prev[t >= d ? 0 : SG + t - d];
+          if (decltype(TAIL)::value && c0 + t >= lim) g = make_float2(0.f, 0.f);
           acc[d][0][0] += u.x * g.x;
           acc[d][0][1] += u.x * g.y;
           acc[d][1][0] += u.y * g.x;
@@ -184,7 +191,10 @@ __global__ __launch_bounds__(512) void k_supervectors(
     }
     b ^= 1;
     if (c0 + SG < steps) weights(us[b], mus[b]);
-  }
+  };
+  int c0 = 0;
+  for (; c0 + SG <= full; c0 += SG) round(std::false_type{}, c0);
+  for (; c0 < steps; c0 += SG) round(std::true_type{}, c0);
   for (int off = 1 << kshift; off < 64; off <<= 1)
 #pragma unroll
     for (int d = 0; d < SG; ++d)

@@ -94,6 +94,37 @@ def test_supervector_spectra_tiles(cuda, n, N, C, ell):
         assert np.all(np.abs(got[ii] - ref) <= (m + 3) * 2.0 ** -24 * mag), ii
 
 
+@pytest.mark.parametrize("n,N,C,ell", [(40, 9, 9, 4), (61, 16, 14, 5), (130, 12, 27, 8), (200, 33, 50, 3),
+                                       (150, 96, 20, 8), (120, 11, 97, 2)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_supervector_spectra_of_non_finite_images(cuda, n, N, C, ell, bad):
+    """A non-finite image reaches the delays whose sums it belongs to and no other: image j is in
+    delay ii for C - 1 - ii <= j < C - 1 - ii + m.  The other delays keep their bits."""
+    import torch
+    from manifoldem_python_amd import _native as nat
+    rng = np.random.default_rng(n)
+    Kh, m = N * (N // 2 + 1), n - C
+    spec = (rng.normal(size=(n, Kh)) + 1j * rng.normal(size=(n, Kh))).astype(np.complex64)
+    ctf = torch.as_tensor(rng.uniform(0.1, 1, (n, Kh)).astype(np.float32), device=cuda)
+    mu = torch.as_tensor(rng.uniform(0.5, 2, (m, ell)), device=cuda)
+
+    def run(x):
+        sv = torch.empty((C, ell, Kh), dtype=torch.complex64, device=cuda)
+        nat.nlsa_supervectors(torch.as_tensor(x, device=cuda), ctf, n, N, C, mu, 5.0, sv)
+        return sv.cpu().numpy()
+
+    want = run(spec)
+    for j in (0, C // 2, n - C // 2 - 1, n - 2, n - 1):
+        x = spec.copy()
+        x[j] = bad * (1 + 1j) if np.isnan(bad) else complex(bad, -bad)
+        got = run(x)
+        for ii in range(C):
+            if C - 1 - ii <= j < C - 1 - ii + m:
+                assert not np.isfinite(got[ii]).any(), (j, ii)
+            else:
+                np.testing.assert_array_equal(got[ii], want[ii], err_msg=str((j, ii)))
+
+
 @pytest.mark.parametrize("npix,q,ncols", [(1, 1, 1), (64, 2, 127), (129, 19, 128), (600, 20, 130),
                                           (2050, 41, 257), (127, 100, 15), (5000, 33, 40)])
 def test_frame_products_on_tiles(cuda, npix, q, ncols):
