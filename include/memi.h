@@ -237,7 +237,7 @@ int memi_plan(const memi_pd_desc* pds_in_host, int npd, int chunks, int gram_til
  * Each half's K range (two segments of Khp elements, 64-byte steps) is split into
  * info->chunks chunks of ceil(2 steps / chunks) steps, the last one shorter; a chunk count
  * that leaves an empty chunk is rejected.  A plan with an automatic split uses as many of its
- * chunks as the K range fills.
+ * chunks as the K range fills (FP32: eight at least, or all of a plan with fewer).
  * variant: Gram kernel schedule, 0 = default; for 128-wide tiles (two workgroups per CU)
  * 1 = prefetch one K step through registers, 2 = prefetch two, 3 = load each K step straight
  * into LDS (global_load_lds) during the previous step's MFMAs (the default); 256-wide tiles

@@ -571,6 +571,7 @@ inline int auto_chunks(int64_t ut, int BT, int least) {
   return best;
 }
 constexpr int kAutoMinSteps = 6;     // least K steps of a chunk of an automatic split
+constexpr int kAutoFp32Chunks = 8;   // chunks that short FP32 operands keep all the same
 
 }  // namespace memi
 
@@ -718,8 +719,14 @@ int memi_ctf_distance(const void* plan_dev, const memi_plan_info* info, const vo
   int64_t spc = (2 * steps + chunks - 1) / chunks;
   int live = chunks;                        // chunks that hold steps
   if (info->auto_split) {
-    // short operands leave some of the plan's chunks empty; a chain stays within a segment
-    spc = std::min<int64_t>(std::max<int64_t>(spc, kAutoMinSteps), steps);
+    // short operands leave some of the plan's chunks empty; a chain stays within a segment, and a
+    // float32 product's (whose rounding is that of its sums alone) within an eighth of the half
+    int64_t most = steps;
+    if (precision == MEMI_PREC_FP32) {
+      const int64_t c = std::min(chunks, kAutoFp32Chunks);
+      most = std::min(most, (2 * steps + c - 1) / c);
+    }
+    spc = std::min<int64_t>(std::max<int64_t>(spc, kAutoMinSteps), most);
     live = (int)((2 * steps + spc - 1) / spc);
   }
   MEMI_CHECK_ARG(steps < (1LL << 29) && (int64_t)(live - 1) * spc < 2 * steps && live <= chunks,

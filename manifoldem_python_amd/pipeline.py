@@ -29,8 +29,9 @@ LOG_EPS = np.arange(-150, 150.2, 0.2)        # DMembeddingII.py:146 (1501 points
 LOG_EPS.setflags(write=False)                # a constant; read-only arrays are cached by identity
 KAPPA = {nat.PREC_FP32: 1.0e4, nat.PREC_SPLIT_BF16: 8.0}
 # default K chunks per Gram half: chosen by the plan from its number of tiles.  FP32 takes at least
-# six, which keeps its float32 sums short (its products carry no split error)
-CHUNKS = {nat.PREC_FP32: -6, nat.PREC_SPLIT_BF16: nat.CHUNKS_AUTO}
+# eight: its products carry no split error, so that its rounding is that of its float32 sums, which
+# grows with their length
+CHUNKS = {nat.PREC_FP32: -8, nat.PREC_SPLIT_BF16: nat.CHUNKS_AUTO}
 GRAM_TILE = 128                                          # default Gram output tile side
 
 

@@ -153,6 +153,15 @@ def test_plan_automatic_split(ns, tile):
             nat.Plan(rows0, ns, ns, chunks=bad, device="cpu", gram_tile=tile)
 
 
+@pytest.mark.parametrize("ns", [[1], [900], [2000], [4000], [400] * 64, [300] * 500])
+def test_default_fp32_split_keeps_eight_chunks(ns):
+    """The default FP32 split never sums over more than an eighth of a half's K range."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    rows0 = np.concatenate(([0], np.cumsum(ns)[:-1]))
+    pl_ = nat.Plan(rows0, ns, ns, chunks=pl.CHUNKS[nat.PREC_FP32], device="cpu")
+    assert pl_.info.chunks >= 8
+
+
 def test_ritz_vectors_checks_meta_on_the_host():
     """A Ritz assembly whose basis length J exceeds the PD size (or k exceeds kmax) is refused
     before launch: the kernel indexes the basis and S by these numbers."""

@@ -281,6 +281,18 @@ def test_gram_automatic_split(cuda, precision, n, N, tile):
     assert np.all(np.diag(D) == 0)
 
 
+@pytest.mark.parametrize("n,N", [(40, 12), (130, 16), (70, 20), (60, 24)])
+def test_gram_fp32_split_of_short_operands(cuda, n, N):
+    """Operands so short that an eighth of a half is under the automatic split's least chunk: the
+    FP32 default still sums over no more than that, the same partial sums as eight chunks."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    s = _setup(n, N, seed=n)
+    geo, out, op = _gpu_prep(s, cuda, 0)
+    D = [pl.ctf_distances(nat.Plan([0], [n], [n], chunks=c), op, out["fy"], out["ctf"], N)
+         .block(0).cpu().numpy() for c in (pl.CHUNKS[0], 8)]
+    np.testing.assert_array_equal(D[0], D[1])
+
+
 def _operand_values(op):
     import torch
     if op.lo is None:
