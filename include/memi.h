@@ -388,7 +388,9 @@ int memi_lanczos_steps_sparse(const void* plan_dev, const memi_plan_info* info,
  * groups: int32 [n_groups][8] on the device, one entry per workgroup: {PD, first row, end row,
  * place in the PD's group, workgroups of the group (at most 64), first workgroup of the group, 0,
  * 0}; the entries of a PD are consecutive and their row ranges cover it.  The caller makes sure
- * that n_groups is at most the number of CUs the stream may use.  max_rows: the largest row
+ * that n_groups workgroups run at once, one per CU: on a CU-masked stream at most the number of
+ * XCDs times the CUs of the XCD that keeps the fewest, since workgroups are dealt to the XCDs in
+ * turn.  max_rows: the largest row
  * range.  W: float64 [m * n_rows], kept between the launches of a run (the columns L v_l).
  * xch: float64 [xch_len >= nsteps (n_rows + n_groups (j0 + nsteps + 3))].  The step's LDS,
  * 8 (max_n + (j0 + nsteps + 4) max_rows + j0 + nsteps + 1100) bytes, is at most

@@ -7,6 +7,7 @@ There is no CPU fallback: if the library is missing or a tensor is on the CPU th
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 import numpy as np
@@ -528,6 +529,31 @@ def cu_masked_stream(keep, device=None):
 
 
 _MASKED_STREAMS = {}
+
+
+@functools.lru_cache(maxsize=64)
+def resident_cus(mask, n_cu):
+    """How many workgroups of one per CU are sure to run at once on a stream with the CU mask
+    (a tuple of 32-bit words): workgroups are dealt to the XCDs in turn, so the XCD with the fewest CUs sets
+    the share of all.  XCDs hold 32 CUs; mask bit i is on XCD i mod their number as the driver
+    enumerates CUs, and the count for an XCD-by-XCD enumeration bounds it too."""
+    bits = [i for i in range(n_cu) if mask[i // 32] >> (i % 32) & 1]
+    n_xcd = max(1, n_cu // 32)
+    few = lambda xcd: min(np.bincount([xcd(i) for i in bits], minlength=n_xcd)[:n_xcd])
+    return n_xcd * int(min(few(lambda i: i % n_xcd), few(lambda i: i // 32 % n_xcd)))
+
+
+def stream_resident_cus(device):
+    """``resident_cus`` of the device's current stream (every CU when it has no mask)."""
+    n_cu = torch.cuda.get_device_properties(device).multi_processor_count
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipExtStreamGetCUMask.argtypes = [c_vp, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32)]
+    nw = (n_cu + 31) // 32
+    mask = (ctypes.c_uint32 * nw)()
+    err = hip.hipExtStreamGetCUMask(c_vp(torch.cuda.current_stream(device).cuda_stream), nw, mask)
+    if err:
+        raise RuntimeError(f"hipExtStreamGetCUMask failed ({err})")
+    return resident_cus(tuple(mask), n_cu)
 
 
 class HipEvents:

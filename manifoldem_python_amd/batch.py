@@ -163,9 +163,6 @@ class OverlappedSteps:
             try:
                 self.main = nat.cu_masked_stream(lambda b: b >= cut)
                 self.side = nat.cu_masked_stream(lambda b: b < cut)
-                cus = torch.cuda.get_device_properties(self.main.device).multi_processor_count
-                for wsp in (wsp_a, wsp_b):       # the embeddings' share of the CUs
-                    wsp.plan.cu_limit = cus * self.split // 32
             except RuntimeError as e:
                 warnings.warn(f"OverlappedSteps: CU-masked streams unavailable ({e}); the two "
                               "streams share all CUs", RuntimeWarning, stacklevel=2)

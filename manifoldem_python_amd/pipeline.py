@@ -613,16 +613,14 @@ def run_groups(ns, work, max_n, cus):
     return out
 
 
-def _run_state(plan, L, m, dev):
+def _run_state(plan, L, m, dev, cus):
     """Buffers of memi_lanczos_run for the plan, or None when its workgroups do not all fit on the
-    CUs (``plan.cu_limit`` of them, when a caller keeps the plan's work on a part of the GPU)."""
+    `cus` CUs that are sure to run one each at once (``nat.stream_resident_cus``)."""
     ns = plan.ns.astype(np.int64)
     per_row = ns.astype(np.float64)
     if isinstance(L, tuple):
         few = plan.ks * SPARSE_RATIO <= ns if len(L) == 5 else np.ones(len(ns), dtype=bool)
         per_row = np.where(few, 3.0 * plan.ks, per_row)   # ~2 k nonzeros of 12 bytes
-    cus = getattr(plan, "cu_limit", None) or \
-        torch.cuda.get_device_properties(dev).multi_processor_count
     table = run_groups(ns, ns * per_row, int(plan.info.max_n), int(cus))
     if table is None:
         return None
@@ -702,8 +700,14 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
             st["summary_h"] = torch.zeros(3 * npd + 1, dtype=torch.float64, pin_memory=True)
             st["summary_ev"] = torch.cuda.Event()
         st["graph"] = None
-        st["run"] = _run_state(plan, L, m, dev) if may_run else None
+        st["run"] = st["cus"] = None
         plan._lanczos = st
+    # the workgroups of memi_lanczos_run are sized for the CUs of the stream in use, which is
+    # another one when a plan is embedded on its own and in overlapped steps
+    cus = nat.stream_resident_cus(dev) if may_run else None
+    if st["cus"] != cus:
+        st["run"], st["cus"] = _run_state(plan, L, m, dev, cus), cus
+        st["summary"][3 * npd:].zero_()          # the abort flag of the table before
     run = st["run"]
     if graph and run is None and st["graph"] is None:
         g = torch.cuda.CUDAGraph()

@@ -605,3 +605,27 @@ def test_lanczos_run_continues_past_its_lds(cuda, monkeypatch):
     res = pl.lanczos_eigs(plan, L, kk)
     assert plan._lanczos["run"] is not None and max(r[2] for r in res) > 16
     _check_eigs(plan, L, res, kk)
+
+
+def test_lanczos_run_follows_the_streams_cus(cuda):
+    """One plan embedded on the whole GPU, on CU-masked streams (an uneven one among them: four XCDs
+    with 8 CUs) and on the whole GPU again: the workgroup table fits what each stream holds, the
+    launches that hold a block of steps stay in use and the eigenpairs are those of eigh."""
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    ns, kk = [150] * 60, [6] * 60
+    plan, L = _kernel(cuda, ns, ns)
+    want = None
+    for split, most in ((32, 256), (16, 128), (12, 64), (32, 256)):
+        st = torch.cuda.current_stream() if split == 32 else \
+            nat.cu_masked_stream(lambda b: b >= 32 - split)
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(st):
+            assert nat.stream_resident_cus(cuda) == most
+            res = pl.lanczos_eigs(plan, L, kk)
+        st.synchronize()
+        run = plan._lanczos["run"]
+        assert run is not None and most // 2 < len(run["groups"]) <= most
+        _check_eigs(plan, L, res, kk)
+        want = want or [r[2] for r in res]
+        assert [r[2] for r in res] == want

@@ -206,3 +206,33 @@ def test_run_groups_refuse_what_does_not_fit():
     from manifoldem_python_amd import pipeline as pl
     for ns, cus in (([4097], 256), ([50] * 300, 256), ([2400] * 40, 256), ([2000], 4)):
         assert pl.run_groups(ns, np.square(ns), max(ns), cus) is None
+
+
+@pytest.mark.parametrize("split,want", [(8, 64), (12, 64), (16, 128), (20, 128), (24, 192), (32, 256)])
+def test_resident_cus_of_a_split(split, want):
+    """Workgroups are dealt to the XCDs in turn, so a CU mask holds eight times what its poorest XCD
+    holds: bits 20..31 of every 32 leave four XCDs 16 CUs and four 8."""
+    from manifoldem_python_amd import _native as nat
+    keep = sum(1 << b for b in range(32 - split, 32))
+    assert nat.resident_cus((keep,) * 8, 256) == want
+
+
+def test_resident_cus_of_other_masks():
+    from manifoldem_python_amd import _native as nat
+    full = 0xFFFFFFFF
+    assert nat.resident_cus((full,) * 7 + (0xFF,), 256) == 64     # one XCD's words cut to 8 CUs
+    assert nat.resident_cus((0xF0000000,) * 8, 256) == 0          # no CU on four XCDs
+    assert nat.resident_cus((full,) * 7 + (0,), 256) == 0
+    assert nat.resident_cus((full,), 32) == 32                    # a single XCD
+
+
+def test_run_table_follows_the_cus():
+    """The workgroup table of a plan is never larger than the CUs given for it."""
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    ns = [150] * 60
+    plan = nat.Plan(150 * np.arange(60), ns, ns, chunks=2, device="cpu")
+    L = torch.empty(0, dtype=torch.float64)
+    sizes = [len(pl._run_state(plan, L, 100, torch.device("cpu"), c)["groups"]) for c in (256, 128, 64)]
+    assert sizes[0] > 128 and 64 < sizes[1] <= 128 and sizes[2] <= 64
+    assert pl._run_state(plan, L, 100, torch.device("cpu"), 32) is None
