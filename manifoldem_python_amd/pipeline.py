@@ -628,7 +628,7 @@ def _run_state(plan, L, m, dev, cus):
     # steps per launch: as many as keep the exchange buffer (emptied before every launch) small
     most = int(max(8, min(40, 500_000 // (plan.info.n_rows + 64 * n_groups) // 8 * 8)))
     last = (nat.LANCZOS_RUN_LDS // 8 - int(plan.info.max_n) - 1100 - 4 * max_rows) // (max_rows + 1)
-    last = min(last, m + most)
+    last = min(last, m)
     return dict(groups=torch.as_tensor(table, device=dev), max_rows=max_rows, most=most, last=last,
                 W=torch.empty(m * plan.info.n_rows, dtype=torch.float64, device=dev),
                 xch=torch.empty(nat.lanczos_run_xch_len(plan, n_groups, last, most),
@@ -709,14 +709,7 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
         st["run"], st["cus"] = _run_state(plan, L, m, dev, cus), cus
         st["summary"][3 * npd:].zero_()          # the abort flag of the table before
     run = st["run"]
-    if graph and run is None and st["graph"] is None:
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
-            nat.lanczos_steps(plan, L, st["V"], m, st["j"], check_every, st["active"],
-                              st["W"], st["ab"], H=st["H"])
-        st["graph"] = g
-    V, W, H, ab, active, j_dev, g = (st["V"], st["W"], st["H"], st["ab"], st["active"], st["j"],
-                                     st["graph"])
+    V, W, H, ab, active, j_dev = (st[q] for q in ("V", "W", "H", "ab", "active", "j"))
     if check == "gpu":
         theta, S_dev, steps_t, res_t, piv = st["theta"], st["S"], st["steps"], st["res"], st["piv"]
     # start vectors (column 0 of every PD's basis): fixed by the seed, so built and uploaded once
@@ -748,24 +741,36 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     if run is not None:
         abort_flag = st["summary"][3 * npd:].view(torch.int32)
 
+    def phases():
+        """Queues check_every steps as one launch per phase, captured on first need."""
+        if not graph:
+            nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
+            return
+        if st["graph"] is None:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
+            st["graph"] = g
+        st["graph"].replay()
+
     def block(j, target):
         """Queues steps from j: a block of check_every, or the blocks up to target in one launch.
         Returns the new step count."""
         if run is not None:
             q = max(1, min(-(-(target - j) // check_every), run["most"] // check_every))
-            if j + q * check_every > run["last"]:
+            if min(m, j + q * check_every) > run["last"]:
                 q = 1
-            nsteps = q * check_every
-            if nsteps <= run["most"] and j + nsteps <= run["last"]:
-                nat.lanczos_run(plan, L, V, run["W"], m, j_dev, j, nsteps, active, ab,
-                                run["groups"], run["max_rows"], run["xch"], abort_flag, RUN_SPIN)
-                return min(m, j + nsteps)
-            # the basis has outgrown the workgroups' LDS: the rest of the run step by step
-            nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
-        elif g is not None:
-            g.replay()
-        else:
-            nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
+            end = min(m, j + q * check_every)
+            if end <= run["last"]:
+                while j < end:               # several launches for a block longer than one
+                    nsteps = min(run["most"], end - j)
+                    nat.lanczos_run(plan, L, V, run["W"], m, j_dev, j, nsteps, active, ab,
+                                    run["groups"], run["max_rows"], run["xch"], abort_flag,
+                                    RUN_SPIN)
+                    j += nsteps
+                return end
+            # the basis has outgrown the workgroups' LDS: the rest of the run phase by phase
+        phases()
         return min(m, j + check_every)
 
     j = 0                            # steps queued on the stream

@@ -629,3 +629,42 @@ def test_lanczos_run_follows_the_streams_cus(cuda):
         _check_eigs(plan, L, res, kk)
         want = want or [r[2] for r in res]
         assert [r[2] for r in res] == want
+
+
+def test_lanczos_run_replays_a_graph_past_its_lds(cuda, monkeypatch):
+    """The steps after a basis has outgrown the workgroups' LDS replay one captured block, in this
+    run and the next, instead of launching each phase from the host."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    made, launch, eager = pl._run_state, nat.lanczos_steps, []
+
+    def small(*a):
+        st = made(*a)
+        st["last"] = 16
+        return st
+
+    monkeypatch.setattr(pl, "_run_state", small)
+    monkeypatch.setattr(nat, "lanczos_steps", lambda *a, **k: (eager.append(1), launch(*a, **k)))
+    ns, kk = [500, 140], [16, 9]
+    plan, L = _kernel(cuda, ns, ns)
+    for _ in range(3):
+        res = pl.lanczos_eigs(plan, L, kk)
+        assert max(r[2] for r in res) > 32 and len(eager) == 1
+        _check_eigs(plan, L, res, kk)
+
+
+@pytest.mark.parametrize("check_every", [8, 13, 64, 200])
+def test_lanczos_run_takes_blocks_of_any_length(cuda, monkeypatch, check_every):
+    """Blocks between checks longer than one launch's steps run as several of them (no launch per
+    phase), with the step counts of the launch-per-phase steps."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    ns, kk = [300, 120, 30], [9, 7, 5]
+    plan, L = _kernel(cuda, ns, ns)
+    want = [r[2] for r in pl.lanczos_eigs(plan, L, kk, split=True, check_every=check_every)]
+    launch, used = nat.lanczos_run, []
+    monkeypatch.setattr(nat, "lanczos_run", lambda *a: (used.append(a[6:8]), launch(*a)))
+    monkeypatch.setattr(nat, "lanczos_steps", None)
+    for _ in range(2):
+        res = pl.lanczos_eigs(plan, L, kk, check_every=check_every)
+        assert used and all(n <= 40 for _, n in used)
+        assert [r[2] for r in res] == want
+        _check_eigs(plan, L, res, kk)
