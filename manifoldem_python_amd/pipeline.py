@@ -14,6 +14,8 @@ psi/mu arithmetic on the (n x nEigs+1) eigenvectors.
 """
 from __future__ import annotations
 
+import contextlib
+import threading
 import warnings
 
 import numpy as np
@@ -652,9 +654,26 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
     steps by default).  graph: the launches of one block of
     check_every steps are captured once in a HIP graph and replayed (the step index lives on
     the device).  With split left open and check "gpu", batches whose workgroups all fit on the
-    GPU at once run each block of steps in one launch instead (memi_lanczos_run), and fall back to
-    the launches above if a wait between its workgroups ever runs out.  Returns a list of (lam, V (n x k) numpy, steps, max residual); with full,
-    also the (n_rows x kmax) array the V are row blocks of."""
+    GPU at once run each block of steps in one launch instead (memi_lanczos_run), which may hold
+    every CU that the stream in use has.  While one call does so, calls of other threads on the same
+    device take the launches above; so does a plan from then on when a wait between its workgroups
+    has run out (their CUs held by something outside this process).  Returns a list of (lam,
+    V (n x k) numpy, steps, max residual); with full, also the (n_rows x kmax) array the V are row
+    blocks of."""
+    with contextlib.ExitStack() as held:
+        return _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, split, check, graph, full)
+
+
+_RUN_LOCKS = {}
+
+
+def _run_lock(dev):
+    """Held by the one call at a time whose memi_lanczos_run launches may fill the device: the
+    workgroups of two such launches would wait for each other's CUs."""
+    return _RUN_LOCKS.setdefault(dev.index, threading.Lock())
+
+
+def _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, split, check, graph, full):
     sparse = isinstance(L, tuple)               # (col, val, cnt) of nat.kernel_ell
     dev = (L[1] if sparse else L).device
     npd = plan.npd
@@ -709,6 +728,12 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
         st["run"], st["cus"] = _run_state(plan, L, m, dev, cus), cus
         st["summary"][3 * npd:].zero_()          # the abort flag of the table before
     run = st["run"]
+    if run is not None:
+        lock = _run_lock(dev)
+        if lock.acquire(blocking=False):
+            held.callback(lock.release)
+        else:
+            run = None                           # for this call
     V, W, H, ab, active, j_dev = (st[q] for q in ("V", "W", "H", "ab", "active", "j"))
     if check == "gpu":
         theta, S_dev, steps_t, res_t, piv = st["theta"], st["S"], st["steps"], st["res"], st["piv"]
@@ -748,7 +773,8 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
             return
         if st["graph"] is None:
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
+            # thread_local: other threads may be in the middle of their embeddings
+            with torch.cuda.graph(g, capture_error_mode="thread_local"):
                 nat.lanczos_steps(plan, L, V, m, j_dev, check_every, active, W, ab, H=H)
             st["graph"] = g
         st["graph"].replay()
@@ -797,11 +823,11 @@ def lanczos_eigs(plan, L, ks, m=None, tol=LANCZOS_TOL, check_every=None, seed=20
                 j = block(j, j + check_every)
             st["summary_ev"].synchronize()
             if run is not None and st["summary_h"][3 * npd:].view(torch.int32)[0]:
-                # a wait between workgroups ran out (work on other streams held their CUs): this
-                # plan goes back to one launch per phase of a step, from the start
+                # a wait between workgroups ran out (something else held their CUs): this plan
+                # goes back to one launch per phase of a step, from the start
                 st["run"] = None
-                return lanczos_eigs(plan, L, ks, m, tol, check_every, seed, None, check, graph,
-                                    full)
+                return _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, None, check,
+                                     graph, full)
             h = st["summary_h"].numpy()[:3 * npd].reshape(3, npd)
             active_h = h[0].astype(np.int32)
             gap, hist, last = _next_check_gap(jc, h[1], h[2], active_h, tol, check_every, hist)
@@ -1047,7 +1073,8 @@ KERNEL_DTYPE = torch.float64
 def dm_embed(plan, D, tune, num_eigs=15, logEps=LOG_EPS, rand=None, a0s=None, mask=None,
              eig="lanczos", timer=None, fit="gpu"):
     """a10-a16 for every PD of the plan.  D: flat float32 device buffer.  Returns a list of
-    DMResult (numpy outputs).  eig: "lanczos" (batched GPU Lanczos) or "dense" (rocSOLVER
+    DMResult (numpy outputs).  eig: "lanczos" (batched GPU Lanczos, whose launches may hold every
+    CU of the current stream; see lanczos_eigs for calls of several threads) or "dense" (rocSOLVER
     syevd on each PD, for checking)."""
     dev = D.device
     info = plan.info

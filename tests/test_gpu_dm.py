@@ -668,3 +668,55 @@ def test_lanczos_run_takes_blocks_of_any_length(cuda, monkeypatch, check_every):
         assert used and all(n <= 40 for _, n in used)
         assert [r[2] for r in res] == want
         _check_eigs(plan, L, res, kk)
+
+
+def test_lanczos_run_is_one_call_at_a_time(cuda, monkeypatch):
+    """While another call holds the device for its workgroups, a call uses the launches per phase,
+    with the same result; afterwards the plan is back on the launches that hold a block of steps."""
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    ns, kk = [300, 120], [9, 7]
+    plan, L = _kernel(cuda, ns, ns)
+    launch, used = nat.lanczos_run, []
+    monkeypatch.setattr(nat, "lanczos_run", lambda *a: (used.append(1), launch(*a)))
+    with pl._run_lock(L.device):
+        a = pl.lanczos_eigs(plan, L, kk)
+    assert not used
+    b = pl.lanczos_eigs(plan, L, kk)
+    assert used and pl._run_lock(L.device).acquire(blocking=False)
+    pl._run_lock(L.device).release()
+    for x, y in zip(a, b):
+        assert x[2] == y[2]
+        np.testing.assert_allclose(x[0], y[0], rtol=0, atol=1e-12)
+    _check_eigs(plan, L, a, kk)
+    _check_eigs(plan, L, b, kk)
+
+
+def test_lanczos_of_two_threads(cuda):
+    """Two threads embed plans that would each fill the GPU, on streams of their own: right results
+    and no wait between workgroups run out."""
+    import threading
+    import torch
+    from manifoldem_python_amd import pipeline as pl
+    ns, kk = [150] * 60, [6] * 60
+    work = []
+    for _ in range(2):
+        plan, L = _kernel(cuda, ns, ns)
+        with pl._run_lock(L.device):             # the captured launches, before the threads start
+            pl.lanczos_eigs(plan, L, kk)
+        work.append((plan, L, torch.cuda.Stream(), []))
+    torch.cuda.synchronize()
+
+    def embed(plan, L, stream, out):
+        with torch.cuda.stream(stream):
+            for _ in range(4):
+                out.append(pl.lanczos_eigs(plan, L, kk))
+
+    threads = [threading.Thread(target=embed, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for plan, L, _, out in work:
+        assert len(out) == 4 and plan._lanczos["run"] is not None
+        for res in out:
+            _check_eigs(plan, L, res, kk)
