@@ -109,7 +109,7 @@ __device__ __forceinline__ double wave_total(double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// Block-wide sum (whole waves, up to 512 threads) of a double; result valid in all threads.
+// Block-wide sum (whole waves; sh holds one value per wave) of a double; result valid in all threads.
 // The wave part by DPP (wave_total): a shuffle-down tree goes through LDS permutes, six
 // dependent round trips per sum.
 __device__ inline double block_sum(double v, double* sh) {

@@ -850,6 +850,38 @@ inline int prep_threads(int N, int64_t n) {
   return n <= 2 * CUS ? 512 : 256;
 }
 
+// An image's outputs do not depend on how many images the call prepares, to the last bit: the
+// statistics are summed as by prep_most_threads threads (the most that prep_threads gives the side),
+// and the recursions are cut into the segments of the fewest (prep_segment_threads).  (Segments for
+// the thread count in use would save few images 1 to 6 %: 200 of 70 x 70, whole call 111 us for 116.)
+constexpr int prep_most_threads(int nmax, int nf) { return nmax > 96 || nf == 96 ? 1024 : 512; }
+constexpr int prep_segment_threads(int nmax, int nf) {
+  return nmax > 128 || nf == 128 ? 1024 : nmax > 96 || nf == 96 ? 512 : 256;
+}
+
+// block_sum over R values per thread: thread t of a block of NT stands for the threads t + r NT of
+// one of R NT
+template <int NT, int R>
+__device__ __forceinline__ double block_sum_of(const double (&v)[R], double* sh) {
+  if constexpr (R == 1) {
+    return block_sum(v[0], sh);
+  } else {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double w[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = wave_total(v[r]);
+    __syncthreads();
+    if (lane == 0)
+#pragma unroll
+      for (int r = 0; r < R; ++r) sh[r * (NT / 64) + wid] = w[r];
+    __syncthreads();
+    double t = 0.0;
+    for (int q = 0; q < R * (NT / 64); ++q) t += sh[q];
+    __syncthreads();
+    return t;
+  }
+}
+
 template <int NMAX, int NF, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(prep_waves(NMAX, NF, NT))))
 void k_prep_images(
@@ -890,7 +922,8 @@ void k_prep_images(
   const float* raw = stack + src[img] * (int64_t)N * N;
   const bool cj = conj != nullptr && conj[img] != 0;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  double s1 = 0.0, s2 = 0.0;
+  constexpr int NV = prep_most_threads(NMAX, NF) / NT;
+  double s1[NV] = {}, s2[NV] = {};
   // every load of this thread in flight at once, then the LDS stores and the statistics
   constexpr int PER = (NMAX * NMAX + NT - 1) / NT;
   const int NNi = N * N;
@@ -910,14 +943,14 @@ void k_prep_images(
       A[r * S + a] = vv[u];
       const int xd = 2 * r - N + 2, yd = 2 * a - N;
       if (xd * xd + yd * yd >= N * N) {
-        s1 += (double)vv[u];
-        s2 += (double)vv[u] * vv[u];
+        s1[u % NV] += (double)vv[u];
+        s2[u % NV] += (double)vv[u] * vv[u];
       }
     }
   }
   const double NN = (double)N * N;
-  const double mean = block_sum(s1, red) / NN;
-  const double sd = sqrt(block_sum(s2, red + 16) / NN - mean * mean);
+  const double mean = block_sum_of<NT>(s1, red) / NN;
+  const double sd = sqrt(block_sum_of<NT>(s2, red + 16) / NN - mean * mean);
   const double inv_sd = 1.0 / sd;
   for (int r = wv; r < N; r += nw)
     for (int c = lane; c < N; c += 64)
@@ -944,13 +977,14 @@ void k_prep_images(
   // segments of the recursions: short chains for small sides (200 images of 48 x 48: 54 us with
   // 8, 58 with 20 samples at least); the others run as fast with 20, restarting less often
   const int seg = N <= 80 ? 8 : 20;
-  bspline_prefilter(A, N, S, zN, seg);
+  constexpr int st = prep_segment_threads(NMAX, NF);
+  bspline_prefilter(A, N, S, zN, seg, st);
   // the rotations run with the side as a run-time value: with every pixel's coordinates
   // constant-folded the compiler computes them all ahead and spills
   int n_rt = N;
   asm volatile("" : "+s"(n_rt));
   spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot1[img]);
-  bspline_prefilter(A, N, S, zN, seg);
+  bspline_prefilter(A, N, S, zN, seg, st);
   spline_sample_inplace<NMAX, 0, NT>(A, n_rt, S, rot2[img]);
   if (img_out) {
     float* o = img_out + img * (int64_t)N * N;

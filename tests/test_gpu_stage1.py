@@ -353,6 +353,29 @@ def test_fused_prep_thread_counts(cuda, n, N):
     assert np.max(np.abs(va - vb)) < 1e-5 * np.max(np.abs(vb))
 
 
+@pytest.mark.parametrize("N", [33, 48, 64, 70, 80, 90, 95, 96, 97, 105, 112, 120, 127, 135])
+def test_fused_prep_does_not_depend_on_the_image_count(cuda, N):
+    """An image's spectrum, operand row and rotated copy have the same bits alone and in calls of any
+    size (the threads per image change at 256, 512 and 1024 images)."""
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl, synth
+    ctf = nat.ctf_params(synth.PIX, synth.CS, synth.EKV, synth.AMPC, np.inf)
+    g = torch.Generator(device=cuda).manual_seed(N)
+    stack = torch.randn(16, N, N, device=cuda, generator=g)
+    want = None
+    for n in (16, 257, 513, 1025):
+        src = torch.arange(n, device=cuda) % 16
+        op = pl.Operand(n, N, 0, cuda)
+        out = pl.prepare_images(stack, src, (src % 3 == 0).to(torch.int32), (src * 7.3 - 50).double(),
+                                torch.full((n,), 31.7, dtype=torch.float64, device=cuda),
+                                (8000 + 300.0 * src).double(), N,
+                                dict(type="Butter", Qc=0.5, N=8), ctf, operand=op)
+        got = [a.reshape(n, -1)[:16].clone() for a in (out["fy"], out["imgAll"], out["ctf"], op.hi)]
+        want = want or got
+        for a, b in zip(got, want):
+            assert torch.equal(a, b), n
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("N", [40, 45, 70, 96, 128, 150, 160])
 def test_fused_prep_matches_staged(cuda, precision, N):
