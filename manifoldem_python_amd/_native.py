@@ -778,11 +778,6 @@ def lanczos_run_xch_len(plan, n_groups, j_end, nsteps):
     return nsteps * (plan.info.n_rows + n_groups * (j_end + 3))
 
 
-def lanczos_run_lds(plan, max_rows, j_end):
-    """Upper bound of memi_lanczos_run's LDS bytes per workgroup for steps that end at j_end."""
-    return 8 * (int(plan.info.max_n) + (j_end + 4) * max_rows + j_end + 1100)
-
-
 def lanczos_run(plan, L, V, Wst, m, j_dev, j0, nsteps, active, ab, groups, max_rows, xch,
                 abort_flag, spin):
     """nsteps Lanczos steps from step j0 in one launch (memi_lanczos_run).  L as in

@@ -134,8 +134,7 @@ struct Dft<7> : DftOdd<7> {};
 // q / d for 0 <= q < 2^21, d >= 1, by the rounded reciprocal inv_d of d: (q + 1/2) / d is at
 // least 1 / (2 d) away from every integer, and the two roundings move it by less than
 // (q / d) 2^-22 < 1 / (2 d)
-__device__ inline int fdivi(int q, int d, float inv_d) {
-  (void)d;
+__device__ inline int fdivi(int q, float inv_d) {
   return (int)(((float)q + 0.5f) * inv_d);
 }
 
@@ -146,7 +145,7 @@ __device__ inline int qdiv(int q, int d, float inv_d) {
   if constexpr (NF > 0)
     return q / d;
   else
-    return fdivi(q, d, inv_d);
+    return fdivi(q, inv_d);
 }
 
 // Every transform below works in ONE LDS buffer.  The line transforms are in-place

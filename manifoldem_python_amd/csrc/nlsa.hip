@@ -343,7 +343,6 @@ __global__ __launch_bounds__(256) void k_gram_cols(const double* __restrict__ U,
 // us; 128 x 128 outputs, one workgroup per CU: 454; the vector units with 4 x 4 outputs per
 // thread, two LDS reads for every two products: 410).
 constexpr int IM_P = 64, IM_J = 128, IM_K = 20;
-typedef double doublex4_t __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256, 2) void k_imgt(const double* __restrict__ U,
                                                  const double* __restrict__ H,

@@ -205,22 +205,21 @@ __global__ void k_hs_derivatives(const float* __restrict__ frames,
 // the image is the nearest edge cell (mode 'reflect' at distance 1).  Used for float32 flows,
 // which round uAvg and every later operation to float32; float64 flows run on k_hs_strips.
 //
-//   uAvg = sum of the 8 neighbours x HSKERN (scipy's raster order, float64, rounded to T)
+//   uAvg = sum of the 8 neighbours x HSKERN (scipy's raster order, float64, rounded to float32)
 //   der  = ((fx uAvg + fy vAvg) + ft) / den,   den = (float)((alpha^2 + fx^2) + fy^2)
-//   U = uAvg - fx der,  V = vAvg - fy der       (in T: float64 for a float64 start, float32 for
-//                                                a float32 start, as numpy promotes)
-template <typename T, int TS, int R, int NT>
+//   U = uAvg - fx der,  V = vAvg - fy der       (in float32, as numpy promotes a float32 start)
+template <int TS, int R, int NT>
 __global__ __launch_bounds__(NT) void k_hs_iterate(
     const float* __restrict__ gfx, const float* __restrict__ gfy, const float* __restrict__ gft,
     int H, int W, int tiles_x, int ntiles, float alpha2, int iters,
-    const T* __restrict__ Uin, const T* __restrict__ Vin, T* __restrict__ Uout,
-    T* __restrict__ Vout) {
+    const float* __restrict__ Uin, const float* __restrict__ Vin, float* __restrict__ Uout,
+    float* __restrict__ Vout) {
 #pragma clang fp contract(off)
   constexpr int E = TS + 2 * R;
   constexpr int NC = E * E;
   constexpr int PER = (NC + NT - 1) / NT;
-  __shared__ T sU[NC];
-  __shared__ T sV[NC];
+  __shared__ float sU[NC];
+  __shared__ float sV[NC];
   __shared__ float sfx[NC];
   __shared__ float sfy[NC];
   __shared__ float sft[NC];
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(NT) void k_hs_iterate(
 
   constexpr double w1 = 1.0 / 12, w2 = 1.0 / 6;
   for (int s = 1; s <= iters; ++s) {
-    T nu[PER], nv[PER];
+    float nu[PER], nv[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int c = threadIdx.x + k * NT;
@@ -276,12 +275,12 @@ __global__ __launch_bounds__(NT) void k_hs_iterate(
         au += (double)sU[c + dn + lf] * w1; av += (double)sV[c + dn + lf] * w1;
         au += (double)sU[c + dn] * w2;      av += (double)sV[c + dn] * w2;
         au += (double)sU[c + dn + rt] * w1; av += (double)sV[c + dn + rt] * w1;
-        const T ua = (T)au, va = (T)av;
+        const float ua = (float)au, va = (float)av;
         const float fx = sfx[c], fy = sfy[c];
         const float den = (alpha2 + fx * fx) + fy * fy;
-        const T der = (((T)fx * ua + (T)fy * va) + (T)sft[c]) / (T)den;
-        nu[k] = ua - (T)fx * der;
-        nv[k] = va - (T)fy * der;
+        const float der = ((fx * ua + fy * va) + sft[c]) / den;
+        nu[k] = ua - fx * der;
+        nv[k] = va - fy * der;
       }
     }
     __syncthreads();
@@ -752,7 +751,7 @@ int memi_hs_iterate(const float* fx, const float* fy, const float* ft, int64_t n
                            W, t, alpha2, it, ui, vi, uo, vo);
       MEMI_CHECK_LAUNCH("k_hs_strips");
     } else {
-      hipLaunchKernelGGL((k_hs_iterate<float, kHsTile, kHsHalo, kHsThreads>), grid,
+      hipLaunchKernelGGL((k_hs_iterate<kHsTile, kHsHalo, kHsThreads>), grid,
                          dim3(kHsThreads), 0, s, fx, fy, ft, H, W, t.nx, (int)ntiles, alpha2, it,
                          (const float*)cur_u, (const float*)cur_v, (float*)nxt_u,
                          (float*)nxt_v);

@@ -1202,8 +1202,7 @@ int memi_prep_images(const float* stack, int64_t n_stack, const int64_t* src,
       else if (N <= 112) MEMI_PREP(112, 0, 512);
       else if (N <= 128 && nt == 1024) MEMI_PREP(128, 0, 1024);
       else if (N <= 128) MEMI_PREP(128, 0, 512);
-      else if (N <= 136 && nt == 1024) MEMI_PREP(136, 0, 1024);
-      else if (N <= 136) MEMI_PREP(136, 0, 512);
+      else if (N <= 136) MEMI_PREP(136, 0, 1024);
       else MEMI_PREP(160, 0, 1024);
   }
 #undef MEMI_PREP
