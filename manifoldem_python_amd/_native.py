@@ -543,14 +543,25 @@ def resident_cus(mask, n_cu):
     return n_xcd * int(min(few(lambda i: i % n_xcd), few(lambda i: i // 32 % n_xcd)))
 
 
+@functools.lru_cache(maxsize=1)
+def _get_cu_mask():
+    f = ctypes.CDLL("libamdhip64.so").hipExtStreamGetCUMask   # loading costs 60 us a time
+    f.argtypes = [c_vp, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32)]
+    return f
+
+
+@functools.lru_cache(maxsize=64)
+def _cu_count(index):
+    return torch.cuda.get_device_properties(index).multi_processor_count
+
+
 def stream_resident_cus(device):
     """``resident_cus`` of the device's current stream (every CU when it has no mask)."""
-    n_cu = torch.cuda.get_device_properties(device).multi_processor_count
-    hip = ctypes.CDLL("libamdhip64.so")
-    hip.hipExtStreamGetCUMask.argtypes = [c_vp, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32)]
+    index = torch.cuda.current_device() if device.index is None else device.index
+    n_cu = _cu_count(index)
     nw = (n_cu + 31) // 32
     mask = (ctypes.c_uint32 * nw)()
-    err = hip.hipExtStreamGetCUMask(c_vp(torch.cuda.current_stream(device).cuda_stream), nw, mask)
+    err = _get_cu_mask()(torch._C._cuda_getCurrentRawStream(index), nw, mask)
     if err:
         raise RuntimeError(f"hipExtStreamGetCUMask failed ({err})")
     return resident_cus(tuple(mask), n_cu)
@@ -778,12 +789,13 @@ def lanczos_run_xch_len(plan, n_groups, j_end, nsteps):
     return nsteps * (plan.info.n_rows + n_groups * (j_end + 3))
 
 
-def lanczos_run(plan, L, V, Wst, m, j_dev, j0, nsteps, active, ab, groups, max_rows, xch,
-                abort_flag, spin):
-    """nsteps Lanczos steps from step j0 in one launch (memi_lanczos_run).  L as in
-    ``lanczos_steps``; groups: int32 (n_groups, 8) device table, one row per workgroup; abort_flag:
-    int32 device tensor, nonzero afterwards when a bounded wait ran out (the run is then
-    unusable)."""
+def lanczos_runner(plan, V, Wst, m, j_dev, active, ab, groups, max_rows, xch, abort_flag, spin):
+    """bind(L) -> launch(j0, nsteps): nsteps Lanczos steps from step j0 in one launch
+    (memi_lanczos_run).  The workspaces are checked here, once for a plan's runs, and the kernel L
+    (as in ``lanczos_steps``) and the current stream in bind, once for the launches of one run: a
+    call from Python costs more than a step of a small PD.  groups: int32 (n_groups, 8) device
+    table, one row per workgroup; abort_flag: int32 device tensor, nonzero afterwards when a bounded
+    wait ran out (the run is then unusable)."""
     I = plan.info
     _need(V.numel() >= m * I.n_rows and Wst.numel() >= m * I.n_rows and
           V.dtype == Wst.dtype == torch.float64 and ab.numel() >= I.n_pd * m * 2 and
@@ -792,23 +804,38 @@ def lanczos_run(plan, L, V, Wst, m, j_dev, j0, nsteps, active, ab, groups, max_r
           "lanczos_run: groups must be int32 (n_groups, 8)")
     _need(xch.dtype == torch.float64 and j_dev.dtype == torch.int32 and j_dev.numel() >= 2 and
           abort_flag.dtype == torch.int32, "lanczos_run: xch float64, j_dev and abort_flag int32")
-    col = val = cnt = sel = Ld = None
-    if isinstance(L, tuple):
-        col, val, cnt = L[:3]
-        if len(L) == 5:
-            sel, Ld = L[3], L[4]
-    else:
-        Ld = L
-    _need(Ld is None or (Ld.numel() >= I.d_elems and
-                         Ld.dtype in (torch.float32, torch.float64)), "lanczos_run: L")
-    _need(sel is None or (sel.dtype == torch.int32 and sel.numel() >= I.n_pd and
-                          Ld.dtype == torch.float64), "lanczos_run: sel")
-    opt = lambda t: None if t is None else _p(t)
-    call("memi_lanczos_run", _p(plan.dev), ctypes.byref(plan.info), opt(Ld),
-         int(Ld is None or Ld.dtype == torch.float64), opt(col), opt(val), opt(cnt), opt(sel),
-         _p(V), _p(Wst), int(m), _p(j_dev), int(j0), int(nsteps), _p(active), _p(ab), _p(groups),
-         int(groups.shape[0]), int(max_rows), _p(xch), int(xch.numel()), _p(abort_flag), int(spin),
-         _stream())
+    fn, info = load().memi_lanczos_run, ctypes.byref(plan.info)
+    kept = (plan.dev, V, Wst, j_dev, active, ab, groups, xch, abort_flag)    # with their addresses
+    pd, pV, pW, pj, pa, pab, pg, px, pf = (_p(t) for t in kept)
+    m, n_groups, max_rows, xlen, spin = (int(q) for q in (m, groups.shape[0], max_rows, xch.numel(),
+                                                          spin))
+
+    def bind(L, kept=kept):
+        col = val = cnt = sel = Ld = None
+        if isinstance(L, tuple):
+            col, val, cnt = L[:3]
+            if len(L) == 5:
+                sel, Ld = L[3], L[4]
+            _need(min(col.numel(), val.numel()) >= I.d_elems and cnt.numel() >= I.n_rows and
+                  col.dtype == cnt.dtype == torch.int32 and val.dtype == torch.float64,
+                  "lanczos_run: sparse rows")
+        else:
+            Ld = L
+        _need(Ld is None or (Ld.numel() >= I.d_elems and
+                             Ld.dtype in (torch.float32, torch.float64)), "lanczos_run: L")
+        _need(sel is None or (sel.dtype == torch.int32 and sel.numel() >= I.n_pd and
+                              Ld.dtype == torch.float64), "lanczos_run: sel")
+        f64 = int(Ld is None or Ld.dtype == torch.float64)
+        pL, pc, pv, pn, ps = (_p(t) for t in (Ld, col, val, cnt, sel))
+        stream = _stream()
+
+        def launch(j0, nsteps):
+            _check(fn(pd, info, pL, f64, pc, pv, pn, ps, pV, pW, m, pj, j0, nsteps, pa, pab, pg,
+                      n_groups, max_rows, px, xlen, pf, spin, stream), "memi_lanczos_run")
+
+        return launch
+
+    return bind
 
 
 RITZ_KMAX = 16

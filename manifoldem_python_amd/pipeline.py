@@ -725,8 +725,13 @@ def _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, split, check, gr
     # another one when a plan is embedded on its own and in overlapped steps
     cus = nat.stream_resident_cus(dev) if may_run else None
     if st["cus"] != cus:
-        st["run"], st["cus"] = _run_state(plan, L, m, dev, cus), cus
-        st["summary"][3 * npd:].zero_()          # the abort flag of the table before
+        r = st["run"] = _run_state(plan, L, m, dev, cus)
+        st["cus"] = cus
+        if r is not None:
+            st["summary"][3 * npd:].zero_()      # the abort flag of the table before
+            r["bind"] = nat.lanczos_runner(plan, st["V"], r["W"], m, st["j"], st["active"], st["ab"],
+                                           r["groups"], r["max_rows"], r["xch"],
+                                           st["summary"][3 * npd:].view(torch.int32), RUN_SPIN)
     run = st["run"]
     if run is not None:
         lock = _run_lock(dev)
@@ -764,7 +769,7 @@ def _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, split, check, gr
     steps = np.minimum(ns, m)
     out = [None] * npd
     if run is not None:
-        abort_flag = st["summary"][3 * npd:].view(torch.int32)
+        launch = run["bind"](L)
 
     def phases():
         """Queues check_every steps as one launch per phase, captured on first need."""
@@ -790,9 +795,7 @@ def _lanczos_eigs(held, plan, L, ks, m, tol, check_every, seed, split, check, gr
             if end <= run["last"]:
                 while j < end:               # several launches for a block longer than one
                     nsteps = min(run["most"], end - j)
-                    nat.lanczos_run(plan, L, V, run["W"], m, j_dev, j, nsteps, active, ab,
-                                    run["groups"], run["max_rows"], run["xch"], abort_flag,
-                                    RUN_SPIN)
+                    launch(j, nsteps)
                     j += nsteps
                 return end
             # the basis has outgrown the workgroups' LDS: the rest of the run phase by phase

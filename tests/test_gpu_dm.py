@@ -660,8 +660,15 @@ def test_lanczos_run_takes_blocks_of_any_length(cuda, monkeypatch, check_every):
     ns, kk = [300, 120, 30], [9, 7, 5]
     plan, L = _kernel(cuda, ns, ns)
     want = [r[2] for r in pl.lanczos_eigs(plan, L, kk, split=True, check_every=check_every)]
-    launch, used = nat.lanczos_run, []
-    monkeypatch.setattr(nat, "lanczos_run", lambda *a: (used.append(a[6:8]), launch(*a)))
+    runner, used = nat.lanczos_runner, []
+
+    def counted(*a):
+        def bind(L, bind=runner(*a)):
+            launch = bind(L)
+            return lambda j, n: (used.append((j, n)), launch(j, n))
+        return bind
+
+    monkeypatch.setattr(nat, "lanczos_runner", counted)
     monkeypatch.setattr(nat, "lanczos_steps", None)
     for _ in range(2):
         res = pl.lanczos_eigs(plan, L, kk, check_every=check_every)
@@ -676,8 +683,12 @@ def test_lanczos_run_is_one_call_at_a_time(cuda, monkeypatch):
     from manifoldem_python_amd import _native as nat, pipeline as pl
     ns, kk = [300, 120], [9, 7]
     plan, L = _kernel(cuda, ns, ns)
-    launch, used = nat.lanczos_run, []
-    monkeypatch.setattr(nat, "lanczos_run", lambda *a: (used.append(1), launch(*a)))
+    runner, used = nat.lanczos_runner, []
+
+    def counted(*a):
+        return lambda L, bind=runner(*a): (used.append(1), bind(L))[1]
+
+    monkeypatch.setattr(nat, "lanczos_runner", counted)
     with pl._run_lock(L.device):
         a = pl.lanczos_eigs(plan, L, kk)
     assert not used
