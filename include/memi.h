@@ -392,7 +392,7 @@ int memi_lanczos_steps_sparse(const void* plan_dev, const memi_plan_info* info,
  * XCDs times the CUs of the XCD that keeps the fewest, since workgroups are dealt to the XCDs in
  * turn.  max_rows: the largest row
  * range.  W: float64 [m * n_rows], kept between the launches of a run (the columns L v_l).
- * xch: float64 [xch_len >= nsteps (n_rows + n_groups (j0 + nsteps + 3))].  The step's LDS,
+ * xch: float64 [xch_len >= nsteps (2 n_rows + n_groups (j0 + nsteps + 3))].  The step's LDS,
  * 8 (max_n + (j0 + nsteps + 4) max_rows + j0 + nsteps + 1100) bytes, is at most
  * MEMI_LANCZOS_RUN_LDS, and PDs have at most 4096 rows; j_dev[0] = min(j0 + nsteps, m) afterwards,
  * as memi_lanczos_steps would leave it.

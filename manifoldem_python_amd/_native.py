@@ -786,7 +786,7 @@ LANCZOS_RUN_GMAX = 64            # workgroups per PD
 
 def lanczos_run_xch_len(plan, n_groups, j_end, nsteps):
     """float64 words of memi_lanczos_run's exchange buffer for steps that end at j_end."""
-    return nsteps * (plan.info.n_rows + n_groups * (j_end + 3))
+    return nsteps * (2 * plan.info.n_rows + n_groups * (j_end + 3))
 
 
 def lanczos_runner(plan, V, Wst, m, j_dev, active, ab, groups, max_rows, xch, abort_flag, spin):

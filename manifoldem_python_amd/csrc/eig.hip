@@ -543,7 +543,10 @@ __global__ void k_step_advance(int32_t* __restrict__ jp) {
 // (v_j itself in a launch's first step, afterwards w' of the step before, not yet divided by beta
 // nor stripped of V h):
 //   y = L u on the own rows, turned into L v_j by linearity, (y - sum_l h_l (L v_l)) / beta, from
-//     the stored columns L v_l (Wst);
+//     the stored columns L v_l (Wst).  Where ||h|| is not small against beta, this would magnify
+//     the columns' rounding from step to step (a kernel of fewer distinct points than steps, whose
+//     w' is noise from some step on: eigenvalues off by 1e-9); v_j itself is published there (a
+//     third exchange) and y = L v_j;
 //   alpha = v_j . y over the group (first exchange);
 //   w' = (y - alpha v_j) - beta_{j-1} v_{j-1}, published (second exchange), and with it the own
 //     rows' parts of h = V^T w' and w'.w';
@@ -571,6 +574,8 @@ constexpr int LR_GMAX = 64;                 // workgroups per group
 constexpr int LR_PARTS = LR_NT / 128;       // threads that share a column's sum over the group
 constexpr int LR_UMAX = 8;                  // elements of u per thread: n <= 4096
 constexpr unsigned long long LR_EMPTY = ~0ull;
+// ||h||^2 / beta^2 above which v_j is exchanged: with ||h|| <= beta / 100 the columns' errors fall
+constexpr double LR_REDO = 1e-4;
 
 struct LrGroup {
   int32_t pd, r0, r1, gi, G, wg0;           // this workgroup's rows; its place in the group; the
@@ -729,6 +734,7 @@ __global__ __launch_bounds__(LR_NT) void k_lanczos_run(
   double* xw = xch + P.row0;                                           // [nsteps][n_rows]
   double* xa = xch + (int64_t)nsteps * n_rows;                         // [nsteps][n_wg]
   double* xh = xa + (int64_t)nsteps * n_wg;                            // [nsteps][n_wg][hs]
+  double* xv = xh + (int64_t)nsteps * n_wg * hs + P.row0;              // [nsteps][n_rows]
   double* Vg = V + (int64_t)m * P.row0;
   double* Wg = Wst + (int64_t)m * P.row0;
   for (int e = tid; e < (j0 + 1) * nr; e += LR_NT) {
@@ -741,6 +747,7 @@ __global__ __launch_bounds__(LR_NT) void k_lanczos_run(
   if (tid == 0) *bad = __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   double bprev = j0 > 0 ? ab[((int64_t)g.pd * m + j0 - 1) * 2 + 1] : 0.0;
   double inv = 1.0;                         // 1 / beta of the step before
+  bool lin = false;                         // u is w' of the step before, not v_j
   __syncthreads();
   for (int j = j0; j < j_end && !*bad; ++j) {
     const int t = j - j0;
@@ -762,7 +769,7 @@ __global__ __launch_bounds__(LR_NT) void k_lanczos_run(
       double a = 0.0;
       for (int i = lane; i < nr; i += 64) {
         double y = yl[i];
-        if (t > 0) {
+        if (lin) {
           y = (y - cw[i]) * inv;
           yl[i] = y;
         }
@@ -843,6 +850,7 @@ __global__ __launch_bounds__(LR_NT) void k_lanczos_run(
     hh = wave_total(hh);
     const double beta = sqrt(fmax(h[j + 1] - hh, 0.0));
     inv = beta > 0.0 ? 1.0 / beta : 0.0;
+    lin = !(hh > LR_REDO * beta * beta);    // the same in the whole group, as h is
     // v_{j+1} and the next step's sum_l h_l (L v_l) on the own rows: sixteen lanes per row
     for (int ib = 0; ib < nr; ib += LR_NT / 16) {
       const int i = ib + (tid >> 4), sub = tid & 15;
@@ -872,6 +880,19 @@ __global__ __launch_bounds__(LR_NT) void k_lanczos_run(
         cw[i] = sw;
         Vl[(j + 1) * nr + i] = x;
         if (j + 1 < m) Vg[(int64_t)(j + 1) * n + g.r0 + i] = x;
+        if (!lin) lr_publish(xv + (int64_t)t * n_rows + g.r0 + i, x);
+      }
+    }
+    if (!lin && j + 1 < j_end) {
+#pragma unroll 1
+      for (int k = tid; k < n; k += LR_NT) {
+        const double* const p[1] = {xv + (int64_t)t * n_rows + k};
+        double v[1];
+        if (!lr_wait<1>(p, v, spin, abort_flag)) {
+          *bad = 1;
+          break;
+        }
+        u[k] = v[0];
       }
     }
     if (g.gi == 0 && tid == 0) {
@@ -1423,7 +1444,7 @@ int memi_lanczos_run(const void* plan_dev, const memi_plan_info* info, const voi
   MEMI_CHECK_ARG(info->max_n <= LR_UMAX * LR_NT, "memi_lanczos_run: PDs of at most %d rows (%d)",
                  LR_UMAX * LR_NT, info->max_n);
   const int hs = j0 + nsteps + 2;
-  const int64_t len = (int64_t)nsteps * (info->n_rows + (int64_t)n_groups * (1 + hs));
+  const int64_t len = (int64_t)nsteps * (2 * info->n_rows + (int64_t)n_groups * (1 + hs));
   MEMI_CHECK_ARG(xch_len >= len, "memi_lanczos_run: exchange buffer %lld < %lld",
                  (long long)xch_len, (long long)len);
   int64_t lds = 8 * ((int64_t)info->max_n + 2 * max_rows + hs + LR_PARTS * 128 + 2 +

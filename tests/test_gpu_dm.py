@@ -731,3 +731,30 @@ def test_lanczos_of_two_threads(cuda):
         assert len(out) == 4 and plan._lanczos["run"] is not None
         for res in out:
             _check_eigs(plan, L, res, kk)
+
+
+@pytest.mark.parametrize("distinct", [3, 4, 6, 8])
+def test_lanczos_run_of_few_distinct_points(cuda, distinct):
+    """Kernels of fewer distinct points than Lanczos steps: from some step on the vectors are noise
+    (||h|| is not small against beta), and the eigenvalues stay those of eigh to float64 rounding
+    (40 steps of a unit-norm kernel: below 1e-13)."""
+    import torch
+    from manifoldem_python_amd import _native as nat, pipeline as pl
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        ns = [60, 150, 241]
+        X = [rng.normal(size=(distinct, 3))[np.arange(n) % distinct] for n in ns]
+        D = [((x[:, None] - x[None]) ** 2).sum(2) for x in X]
+        plan = nat.Plan(np.concatenate(([0], np.cumsum(ns)[:-1])), ns, ns, chunks=1)
+        flat = torch.as_tensor(np.concatenate([d.astype(np.float32).ravel() for d in D]),
+                               device=cuda)
+        L = torch.empty(plan.info.d_elems, dtype=torch.float64, device=cuda)
+        deg = torch.empty(2 * plan.info.n_rows, dtype=torch.float64, device=cuda)
+        nat.markov_normalize(plan, flat, pl.knn_mask(plan, flat),
+                             torch.ones(3, dtype=torch.float64, device=cuda), L, deg)
+        res = pl.lanczos_eigs(plan, L, [9] * 3)
+        assert plan._lanczos["run"] is not None
+        for p in range(3):
+            w = np.linalg.eigvalsh(plan.block(L, p).cpu().numpy())
+            w = np.sort(w[np.argsort(-np.abs(w), kind="stable")[:9]])[::-1]
+            np.testing.assert_allclose(res[p][0], w, rtol=0, atol=1e-13)
