@@ -42,6 +42,7 @@ FILTER = dict(type="Butter", Qc=0.5, N=8)
 PEAK_BF16_TFLOPS = 2500.0
 PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
+PEAK_FP64_VECTOR_TFLOPS = 78.6
 
 
 def parse():
@@ -138,7 +139,7 @@ def optflow_only(spec, steps, warmup, with_cpu):
         optflow.movie_flows(movies, 5, "HS")
     torch.cuda.synchronize()
     t_step = (time.perf_counter() - t0) / steps
-    # the Horn-Schunck kernel alone: 200 iterations = 50 launches of 4 fused iterations
+    # the Horn-Schunck iterations alone (k_hs_strips; launches as its tiling needs)
     A = -(-F // 5)
     nP = M * A
     fr = movies[:, ::5].reshape(nP, dim, dim).contiguous()
@@ -155,21 +156,20 @@ def optflow_only(spec, steps, warmup, with_cpu):
         nat.hs_iterate(fx, fy, ft, 2.0, 200, U, V, tu, tv)
     b.record()
     torch.cuda.synchronize()
-    launches = steps * 50
-    us_launch = 1e3 * a.elapsed_time(b) / launches
-    # algorithmic bytes of one launch (4 fused iterations): U, V read and written once in
-    # float64 and fx, fy, ft read once in float32 -- 44 B per pixel of every frame pair
-    alg = nP * dim * dim * 44.0
-    ach = alg / (us_launch * 1e-6) / 1e9
+    us = 1e3 * a.elapsed_time(b) / steps
+    # float64 operations of one cell and iteration: the separable average of U and V (7 each), the
+    # residual's two fmas and the two updates' -- 22 flop
+    alg = nP * dim * dim * 200 * 22.0
+    ach = alg / (us * 1e-6) / 1e12
     line = {"metric": "optical_flow_movies_per_s", "value": M / t_step, "unit": "movies/s",
             "n_gpus": 1, "steps": steps, "warmup": warmup, "ms_per_step": 1e3 * t_step,
             "higher_is_better": True, "dtype": "f64 (flow), f32 (images)", "data": "synthetic",
             "config": {"workload": "optflow_hs", "movies": M, "frames": F, "image": dim,
                        "frame_pairs": nP, "hs_iterations": 200, "block_size_avg": 5},
-            "roofline": {"kernel": "k_hs_iterate<double,32,4,256>", "bound": "hbm",
-                         "achieved": ach, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                         "frac": ach / PEAK_HBM_GBS, "traffic": None,
-                         "us_per_launch": us_launch, "alg_bytes_per_launch": alg}}
+            "roofline": {"kernel": "k_hs_strips", "bound": "valu_f64", "achieved": ach,
+                         "peak": PEAK_FP64_VECTOR_TFLOPS, "unit": "TFLOP/s",
+                         "frac": ach / PEAK_FP64_VECTOR_TFLOPS, "traffic": None,
+                         "us_per_200_iterations": us, "alg_flops": alg}}
     if with_cpu:
         from oracle import optflow as oof
         mv = movies[0].reshape(F, dim * dim).cpu().numpy()

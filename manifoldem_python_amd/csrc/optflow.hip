@@ -4,10 +4,13 @@
 //
 // Reference: CC/hornschunck_simple.py:9-84, CC/OpticalFlowMovie.py:21-24, 202-341, 385-555.
 //
-// Every kernel reproduces the reference's arithmetic: float32 where numpy computes in float32
+// The kernels reproduce the reference's arithmetic: float32 where numpy computes in float32
 // (the diffusion, the derivative images, the denominator alpha^2 + fx^2 + fy^2), float64
 // accumulation rounded once to the output type where scipy.ndimage filters (it accumulates each
 // output in double), and the reference's operation order with floating-point contraction off.
+// Two take another order: the float64 Horn-Schunck iterations (k_hs_strips: a separable average by
+// fma and no division; within 1e-13 of the flow's scale after 200 iterations) and the quotients by
+// constants in the diffusion (products with float64 reciprocals, the same float32 values).
 // Boundaries are scipy's mode 'reflect' (half-sample mirror), which at distance 1 is a clamp.
 //
 // Data layout: a batch of movies is (movie, frame, row, column) row-major; each frame is the
@@ -318,11 +321,14 @@ __global__ __launch_bounds__(NT) void k_hs_iterate(
 // NW waves stack to a band of NW S rows.  A band that does not hold the whole image keeps a halo
 // of `iters` rows (and columns) on each open side, whose cells go stale one per iteration.
 //
-// Bound: float64 issue (16 float64 instructions and 4 to 8 register moves per cell and iteration)
-// and, between launches, 44 B per pixel of U, V, fx, fy, ft.  Eight cells per lane at 10
-// registers each leave four waves per SIMD, which hide the barrier and the row exchange: 640
-// pairs of 128 x 128, 200 iterations take 3.78 ms (16 cells and two waves per SIMD: 3.96; the
-// LDS-tile form above, which reads 16 float64 neighbours per cell from LDS and divides: 11.6).
+// Bound: neither the vector units nor memory alone.  At 128 x 128 the SIMDs issue vector
+// instructions on 56 % of their cycles (64 % of those in float64, the rest register moves), and a
+// launch moves 0.39 GB of U, V, fx, fy, ft, a quarter of its 0.30 ms at a large copy's rate; the
+// 128 KB of LDS leave one workgroup per CU, so nothing runs beside a tile's loads, stores and
+// barriers.  Eight cells per lane at 10 registers each leave four waves per SIMD: 640 pairs of
+// 128 x 128, 200 iterations take 3.85 ms in 13 launches of three tiles per pair (16 cells and two
+// waves per SIMD: 3.96; the LDS-tile form above, which reads 16 float64 neighbours per cell from LDS
+// and divides: 11.6).
 // Two columns per lane halve the DPP moves (one column: 4.08 ms), one suits narrow images; three
 // (5 rows, 40-row bands) were slower at 128 columns (6.9 ms) and at 160 (9.2 against 8.7).
 constexpr int kHsWaves = 16;
